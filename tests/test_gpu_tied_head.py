@@ -126,3 +126,50 @@ def test_one_hot_hidden_rows_select_embedding_columns(sampler):
     ids, _, _, lg = _run(sampler, hidden, embed, prm, seeds)
     assert np.array_equal(lg, embed[:, cols].T)
     assert np.array_equal(ids, np.argmax(embed[:, cols], axis=0).astype(np.uint32))
+
+
+# Both sides of every line the launch draws (rows, 16- and 32-row tiles, the
+# GEMV's output limit) and of every tile: rows, outputs and chunks.
+@pytest.mark.parametrize("B,V,h", [
+    (1, 33, 0), (1, 31, 4), (1, 16385, 129), (2, 1000, 1027), (2, 33, 127), (3, 16384, 36), (3, 16388, 40), (4, 65, 1156),
+    (4, 16385, 32), (5, 64, 33), (16, 65, 35), (17, 63, 64), (32, 129, 31), (33, 4100, 68), (48, 32768, 12),
+    (49, 32768, 8), (63, 32769, 37), (64, 32767, 100), (65, 70001, 5), (96, 2049, 64), (128, 16353, 63)])
+def test_kernel_boundaries(sampler, B, V, h):
+    rs = np.random.default_rng(B * 131 + V + h)
+    hidden, embed = _case(rs, B, V, h, scale=0.3)
+    prm = make_params(0.9, 20, 0.9, 0.02, 1.0)
+    seeds = rs.integers(0, 2**63, size=B, dtype=np.uint64)
+    _check(_run(sampler, hidden, embed, prm, seeds), hidden, embed, prm, seeds)
+
+
+@pytest.mark.parametrize("B", [1, 4, 20, 64])
+def test_rows_off_16_byte_alignment_and_extreme_products(sampler, B):
+    """Both operands start 4 bytes past a 16-byte boundary with odd strides,
+    and the values span products that are denormal, underflow to zero or are
+    of denormal inputs: every kernel's products round as binary32 multiplies."""
+    import torch
+
+    rs = np.random.default_rng(77 + B)
+    V, h = 33000, 130
+    ex = lambda n: np.ldexp(rs.standard_normal(n), rs.integers(-80, -55, size=n)).astype(np.float32)  # noqa: E731
+    hidden, embed = ex((B, h)), ex((V, h))
+    hidden[:, ::7] = np.ldexp(hidden[:, ::7], -75)  # denormals
+    embed[:, ::7] = np.ldexp(embed[:, ::7], 120)
+    dev = torch.device("cuda:0")
+
+    def place(x, ld):
+        buf = torch.zeros(1 + x.shape[0] * ld, dtype=torch.float32, device=dev)
+        view = buf[1:].view(x.shape[0], ld)[:, :x.shape[1]]
+        view.copy_(torch.from_numpy(x))
+        return view
+
+    d_hidden, d_embed = place(hidden, h + 1), place(embed, h + 3)
+    seeds = rs.integers(0, 2**63, size=B, dtype=np.uint64)
+    rng = torch.from_numpy(seeds.view(np.int64).copy()).to(dev)
+    ids = torch.zeros(B, dtype=torch.int32, device=dev)
+    lg = torch.empty(B, V, dtype=torch.float32, device=dev)
+    sampler.sample_tied_head_device(d_hidden, d_embed, make_params(0.0, 1, 1.0, 0.0, 1.0), rng, ids, out_logits=lg)
+    torch.cuda.synchronize()
+    want = oracle.linear_fwd(hidden, embed, threads=8)
+    assert np.count_nonzero(want) > 0
+    assert np.array_equal(lg.cpu().numpy(), want)
