@@ -3,5 +3,5 @@
 #include "fast_kernel.h"
 
 namespace llmhip {
-template hipError_t launch_fast_nch<8, false>(const SampleArgs&, bool, bool, hipStream_t);
+template hipError_t launch_fast_nch<8, false>(const SampleArgs&, bool, hipStream_t);
 }  // namespace llmhip

@@ -1,5 +1,5 @@
 // Register path of the gfx950 sampler: one row per 1024-thread workgroup,
-// V <= 32768, 0 < top_k <= 4096 (and greedy rows).
+// 4 <= V <= 32768, 0 < top_k <= 4096 (and greedy rows).
 //
 // Row semantics: crates/llm-core/src/generate.rs:325-420. The row is read
 // once from HBM into registers, all of it at once (the memory queues run
@@ -563,12 +563,15 @@ __device__ __forceinline__ void rank_in_lds(uint64_t* ord, uint64_t* tmp, uint32
 // BIGK: some top-k row of the call has K > 64. Without it the kernel holds
 // only the small-K rank and tail (a smaller kernel), and a row with more
 // than 512 candidates goes to the general path.
-template <int NCH, bool VEC, bool GREEDY, bool CMODE, bool BIGK>
+template <int NCH, bool GREEDY, bool CMODE, bool BIGK>
 __device__ __forceinline__ bool fast_row(const SampleArgs& a, FastLds<NCH, BIGK>& L) {
   constexpr uint32_t kEnt = FastLds<NCH, BIGK>::kEnt;
   static_assert(sizeof(FastLds<NCH, BIGK>) <= 160u * 1024u, "LDS");
   static_assert(NCH * 4 <= 32, "slot masks are 32 bits");
-  typedef float f4v __attribute__((ext_vector_type(4)));
+  // Rows need no alignment beyond a float's: gfx950's 16-byte global loads
+  // take any 4-byte aligned address (256 rows of 31999 floats: 16.7 us with
+  // a load per value, 10.3 with these; of 32000 floats 10.2).
+  typedef float f4v __attribute__((ext_vector_type(4), aligned(4)));
 
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
@@ -586,8 +589,8 @@ __device__ __forceinline__ bool fast_row(const SampleArgs& a, FastLds<NCH, BIGK>
   const uint32_t b = launch_row(a);
   LLMHIP_MARK(0);
 
-  // Every global load below is issued unconditionally (positions past V and
-  // absent inputs read a valid dummy address), so each wait in the compiled
+  // Every global load below is issued unconditionally (float4s that pass V
+  // read the row's last four floats, absent inputs a valid dummy address), so each wait in the compiled
   // code names exactly the loads it needs. A wave's loads complete at a
   // limited rate (a CU holds only part of its 128 KiB row in flight, and a
   // wave stalls at a load until earlier data has returned), so every wave
@@ -622,16 +625,11 @@ __device__ __forceinline__ bool fast_row(const SampleArgs& a, FastLds<NCH, BIGK>
   float x[NCH * 4];
   auto load_chunk = [&](int c) __attribute__((always_inline)) {
     const uint32_t base = chunk_pos<NCH>((uint32_t)c, wave, lane);
-    if (VEC) {
-      const f4v q = __builtin_nontemporal_load(reinterpret_cast<const f4v*>(row + (base < V ? base : 0u)));
-      x[4 * c + 0] = q.x;
-      x[4 * c + 1] = q.y;
-      x[4 * c + 2] = q.z;
-      x[4 * c + 3] = q.w;
-    } else {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) x[4 * c + j] = __builtin_nontemporal_load(row + (base + j < V ? base + j : 0u));
-    }
+    const f4v q = __builtin_nontemporal_load(reinterpret_cast<const f4v*>(row + min(base, V - 4u)));
+    x[4 * c + 0] = q.x;
+    x[4 * c + 1] = q.y;
+    x[4 * c + 2] = q.z;
+    x[4 * c + 3] = q.w;
   };
   constexpr int NB0 = NCH >= 2 ? 2 : 1;
 #pragma unroll
@@ -682,10 +680,18 @@ __device__ __forceinline__ bool fast_row(const SampleArgs& a, FastLds<NCH, BIGK>
 
   // Positions past V (in the one chunk that straddles V, or in chunks
   // wholly past it) become -inf before their first use: no value at or
-  // above a threshold, never a maximum. The test is uniform per wave.
+  // above a threshold, never a maximum. The test is uniform per wave. The
+  // float4 that straddles V was loaded from V - 4: its values move down.
   auto prep = [&](int c) __attribute__((always_inline)) {
     if ((chunk_block<NCH>((uint32_t)c, wave) + 1u) * 256u > V) {
       const uint32_t base = chunk_pos<NCH>((uint32_t)c, wave, lane);
+      if (V & 3u) {
+        const uint32_t sh = base < V && base + 4u > V ? base + 4u - V : 0u;
+        const float v0 = x[4 * c], v1 = x[4 * c + 1], v2 = x[4 * c + 2], v3 = x[4 * c + 3];
+        x[4 * c + 0] = sh == 0u ? v0 : sh == 1u ? v1 : sh == 2u ? v2 : v3;
+        x[4 * c + 1] = sh == 0u ? v1 : sh == 1u ? v2 : v3;
+        x[4 * c + 2] = sh == 0u ? v2 : v3;
+      }
 #pragma unroll
       for (int j = 0; j < 4; ++j) x[4 * c + j] = base + j < V ? x[4 * c + j] : -INFINITY;
     }

@@ -24,14 +24,14 @@
 static __device__ __align__(256) uint32_t scratch[LLMHIP_NOALLOC_SCRATCH_BYTES / sizeof(uint32_t)];
 
 namespace llmhip {
-hipError_t launch_fast(const SampleArgs& a, bool vec, bool bigk, hipStream_t s);
-hipError_t launch_fast_counts(const SampleArgs& a, bool vec, bool bigk, hipStream_t s);
+hipError_t launch_fast(const SampleArgs& a, bool bigk, hipStream_t s);
+hipError_t launch_fast_counts(const SampleArgs& a, bool bigk, hipStream_t s);
 hipError_t launch_general(const SampleArgs& a, hipStream_t s);
 hipError_t launch_vocab(const SampleArgs& a, bool plain, hipStream_t s);
 hipError_t launch_slotmask(const SampleArgs& a, uint32_t* out, hipStream_t s);
 hipError_t launch_seen_bits(const uint32_t* tokens, uint64_t n, uint32_t V, uint32_t* bits, hipStream_t s);
 hipError_t launch_take_status(uint32_t* words, hipStream_t s);
-hipError_t launch_stream(const SampleArgs& a, bool vec, bool bigk, hipStream_t s);
+hipError_t launch_stream(const SampleArgs& a, bool bigk, hipStream_t s);
 hipError_t launch_read_floor(const float* logits, uint64_t ld, uint32_t B, uint32_t V, int read, float* out,
                              hipStream_t s);
 hipError_t launch_tied_head(const float* hidden, uint64_t ldh, const float* embed, uint64_t lde, float* logits,
@@ -238,11 +238,13 @@ int enqueue(llmhip_ctx* ctx, const float* logits, size_t B, size_t V, size_t ld,
     penalized = penalized || p.repetition_penalty != 1.0f;
     if (b < kRowClsRows) row_cls[b >> 4] |= (uint32_t)__builtin_ctz(c) << ((b & 15u) * 2u);
   }
-  const bool fast_ok = V <= kMaxFastV;
+  // (A row of fewer than four logits has no float4 for the register path to
+  // load: the sorting path takes it.)
+  const bool fast_ok = V >= 4 && V <= kMaxFastV;
   const uint32_t fast_mask = fast_ok ? (classes & (kClassGreedy | kClassTopK)) : 0u;
   // Top-k rows past the register path's V stream through the persistent
   // kernel; full-vocabulary rows take the bucketed exact-fold kernel.
-  const uint32_t stream_mask = fast_ok ? 0u : (classes & kClassTopK);
+  const uint32_t stream_mask = V > kMaxFastV ? (classes & kClassTopK) : 0u;
   const uint32_t vocab_mask = classes & kClassVocab;
   const uint32_t general_mask = classes & ~fast_mask & ~vocab_mask & ~stream_mask;
 
@@ -301,9 +303,6 @@ int enqueue(llmhip_ctx* ctx, const float* logits, size_t B, size_t V, size_t ld,
   }
 
   if (out_probs) HIP_TRY(hipMemsetAsync(out_probs, 0, B * V * sizeof(float), s));
-  // 128-bit row loads need 16-byte aligned rows and V % 4 == 0 (a row's
-  // last float4 must not extend past its V logits).
-  const bool vec = (reinterpret_cast<uintptr_t>(logits) % 16 == 0) && (ld % 4 == 0) && (V % 4 == 0);
   if (fast_mask) {
     if (a.allowed || a.allowed_bits) {
       uint32_t* sm = ws ? ws->slotmask : nullptr;
@@ -315,13 +314,11 @@ int enqueue(llmhip_ctx* ctx, const float* logits, size_t B, size_t V, size_t ld,
       a.slotmask = sm;
     }
     a.row_class_mask = fast_mask;
-    HIP_TRY(a.counts ? launch_fast_counts(a, vec, bigk, s) : launch_fast(a, vec, bigk, s));
+    HIP_TRY(a.counts ? launch_fast_counts(a, bigk, s) : launch_fast(a, bigk, s));
   }
   if (stream_mask) {
-    // A row's last float4 may pass V (the stride is a multiple of 4).
-    const bool svec = (reinterpret_cast<uintptr_t>(logits) % 16 == 0) && (ld % 4 == 0);
     a.row_class_mask = stream_mask;
-    HIP_TRY(launch_stream(a, svec, bigk, s));
+    HIP_TRY(launch_stream(a, bigk, s));
   }
   if (vocab_mask) {
     a.row_class_mask = vocab_mask;

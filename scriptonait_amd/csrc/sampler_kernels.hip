@@ -116,8 +116,8 @@ hipError_t launch_slotmask(const SampleArgs& a, uint32_t* out, hipStream_t s) {
 }
 
 // Calls without a count table (decode steps with one: fast_counts.hip).
-hipError_t launch_fast(const SampleArgs& a, bool vec, bool bigk, hipStream_t s) {
-  return launch_fast_mode<false>(a, vec, bigk, s);
+hipError_t launch_fast(const SampleArgs& a, bool bigk, hipStream_t s) {
+  return launch_fast_mode<false>(a, bigk, s);
 }
 
 hipError_t launch_seen_bits(const uint32_t* tokens, uint64_t n, uint32_t V, uint32_t* bits, hipStream_t s) {

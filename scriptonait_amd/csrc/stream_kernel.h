@@ -8,24 +8,26 @@
 
 namespace llmhip {
 
-template <bool VEC, bool FULL, bool BIGK>
+template <bool TAIL, bool FULL, bool BIGK>
 __global__ __launch_bounds__(kBlock) void sample_stream_kernel(SampleArgs a) {
   __shared__ StreamKernelLds L;
-  stream_rows<VEC, FULL, BIGK>(a, L);
+  stream_rows<TAIL, FULL, BIGK>(a, L);
 }
 
-// One persistent workgroup per CU (at most one per row). vec: rows 16-byte
-// aligned with a stride of a multiple of 4 floats.
+// One persistent workgroup per CU (at most one per row).
 template <bool BIGK>
-hipError_t launch_stream_k(const SampleArgs& a0, bool vec, hipStream_t s) {
+hipError_t launch_stream_k(const SampleArgs& a0, hipStream_t s) {
   SampleArgs a = a0;
   a.launch_rows = launch_grid(a);
   if (a.launch_rows == 0) return hipSuccess;
   const uint32_t grid = std::min(a.launch_rows, std::max(a.cus, 1u));
   const bool full = a.allowed || a.allowed_bits || a.ring_cap;
-  if (vec && full) {
+  // A row's last float4 may pass V where it then still lies in the row's
+  // 16-byte aligned stride; elsewhere it could pass the end of the buffer.
+  const bool tail = a.V % 4u != 0u && (reinterpret_cast<uintptr_t>(a.logits) % 16u != 0u || a.ld % 4u != 0u);
+  if (tail && full) {
     hipLaunchKernelGGL((sample_stream_kernel<true, true, BIGK>), dim3(grid), dim3(kBlock), 0, s, a);
-  } else if (vec) {
+  } else if (tail) {
     hipLaunchKernelGGL((sample_stream_kernel<true, false, BIGK>), dim3(grid), dim3(kBlock), 0, s, a);
   } else if (full) {
     hipLaunchKernelGGL((sample_stream_kernel<false, true, BIGK>), dim3(grid), dim3(kBlock), 0, s, a);
@@ -35,7 +37,7 @@ hipError_t launch_stream_k(const SampleArgs& a0, bool vec, hipStream_t s) {
   return hipGetLastError();
 }
 
-extern template hipError_t launch_stream_k<false>(const SampleArgs&, bool, hipStream_t);
-extern template hipError_t launch_stream_k<true>(const SampleArgs&, bool, hipStream_t);
+extern template hipError_t launch_stream_k<false>(const SampleArgs&, hipStream_t);
+extern template hipError_t launch_stream_k<true>(const SampleArgs&, hipStream_t);
 
 }  // namespace llmhip

@@ -97,9 +97,6 @@ __device__ __forceinline__ uint32_t stream_count(const StreamLds& L, uint32_t id
   return 0u;
 }
 
-// Loads piece p of a row into buf: slot c of thread t holds float4 index
-// p * kSPieceQ + c * kBlock + t (coalesced per slot). Slots past the row read
-// its first float4 (a valid address); prep() marks them excluded.
 // The thread's index, as a value the compiler cannot merge with another
 // use: the per-slot positions derived from it are then recomputed where they
 // are needed rather than held in registers across the row loop.
@@ -109,40 +106,42 @@ __device__ __forceinline__ uint32_t opaque_tid() {
   return t;
 }
 
-template <bool VEC>
-__device__ __forceinline__ void stream_load(float (&buf)[kSNS * 4], const float* row, uint32_t V, uint32_t p) {
-  typedef float f4v __attribute__((ext_vector_type(4)));
+// Loads piece p of a row into buf: slot c of thread t holds float4 index
+// p * kSPieceQ + c * kBlock + t (coalesced per slot). Slots past the row's VL
+// values (V, or V & ~3 with TAIL) read its first float4 (a valid address), and
+// prep() marks them excluded. Rows need no alignment beyond a float's: gfx950's
+// 16-byte global loads take any 4-byte aligned address. 1024 rows of 50257
+// floats, which start at every alignment, top_k 50: 113.4 us with a load per
+// value, 71 with these; rows of 50260 floats take 59.5.
+__device__ __forceinline__ void stream_load(float (&buf)[kSNS * 4], const float* row, uint32_t VL, uint32_t p) {
+  typedef float f4v __attribute__((ext_vector_type(4), aligned(4)));
   const uint32_t tid = opaque_tid();
 #pragma unroll
   for (int c = 0; c < (int)kSNS; ++c) {
     const uint32_t i = 4u * (p * kSPieceQ + (uint32_t)c * kBlock + tid);
-    if (VEC) {
-      const f4v q = __builtin_nontemporal_load(reinterpret_cast<const f4v*>(row + (i < V ? i : 0u)));
-      buf[4 * c + 0] = q.x;
-      buf[4 * c + 1] = q.y;
-      buf[4 * c + 2] = q.z;
-      buf[4 * c + 3] = q.w;
-    } else {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) buf[4 * c + j] = __builtin_nontemporal_load(row + (i + j < V ? i + j : 0u));
-    }
+    const f4v q = __builtin_nontemporal_load(reinterpret_cast<const f4v*>(row + (i < VL ? i : 0u)));
+    buf[4 * c + 0] = q.x;
+    buf[4 * c + 1] = q.y;
+    buf[4 * c + 2] = q.z;
+    buf[4 * c + 3] = q.w;
   }
 }
 
-// The rows of one launch (all threads). VEC: 16-byte aligned rows with a
-// stride of a multiple of 4 floats (a row's last float4 may pass V, not ld).
-// FULL: the call has an allowed mask or is a decode step (a ring, maybe a
-// count table); the other calls run a variant compiled without that code,
-// whose loop keeps fewer values live. BIGK: some row of the launch has
-// K > 64; without it the kernel holds only the register rank and tail, and a
-// row listing more than 512 values is handed over.
-template <bool VEC, bool FULL, bool BIGK>
+// The rows of one launch (all threads). TAIL: the last float4 of the last row
+// could pass the buffer's end, so every row's last V % 4 values are taken one
+// by one (one more register through the loop: it cost the other calls 0.6-2.7%
+// in a kernel for all). FULL: the call has an allowed mask or is a decode step
+// (a ring, maybe a count table); the other calls run a variant compiled without
+// that code, whose loop keeps fewer values live. BIGK: some row of the launch
+// has K > 64; without it the kernel holds only the register rank and tail, and
+// a row listing more than 512 values is handed over.
+template <bool TAIL, bool FULL, bool BIGK>
 __device__ __forceinline__ void stream_rows(const SampleArgs& a, StreamKernelLds& U) {
   StreamLds& L = U.s;
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
-  const uint32_t V = a.V, nrows = a.launch_rows, step = gridDim.x;
-  const uint32_t nq = (V + 3u) / 4u;
+  const uint32_t V = a.V, VL = TAIL ? V & ~3u : V, nrows = a.launch_rows, step = gridDim.x;
+  const uint32_t nq = (VL + 3u) / 4u;
   // Pieces per row, rounded up to even (a piece wholly past V is read as
   // its row's first float4 and excluded): the pieces alternate between the
   // two buffers, and every row starts with piece 0 in A and piece 1 in Bf.
@@ -156,12 +155,14 @@ __device__ __forceinline__ void stream_rows(const SampleArgs& a, StreamKernelLds
     llmhip_params P;
     uint64_t rng0;
     uint32_t h0, h1, done;
+    float last;  // value VL + (thread) of the row, in threads below V - VL
   };
   auto row_info = [&](uint32_t rb) __attribute__((always_inline)) {
     RowInfo r;
     r.P = load_params(a, rb);
     r.rng0 = a.rng_state[rb];
     r.h0 = r.h1 = r.done = 0u;
+    r.last = TAIL ? a.logits[(size_t)rb * a.ld + min(VL + tid, V - 1u)] : 0.0f;
     if (FULL && a.ring_cap) {
       r.h0 = a.ring_len[rb];
       r.h1 = ring_avail(a, rb, r.h0);
@@ -177,8 +178,8 @@ __device__ __forceinline__ void stream_rows(const SampleArgs& a, StreamKernelLds
   uint32_t j = blockIdx.x;
   uint32_t b = launch_row_at(a, j);
   RowInfo ri = row_info(b);
-  stream_load<VEC>(A, a.logits + (size_t)b * a.ld, V, 0u);
-  stream_load<VEC>(Bf, a.logits + (size_t)b * a.ld, V, 1u);
+  stream_load(A, a.logits + (size_t)b * a.ld, VL, 0u);
+  stream_load(Bf, a.logits + (size_t)b * a.ld, VL, 1u);
 
   while (true) {
     const uint32_t jn = j + step;
@@ -261,15 +262,15 @@ __device__ __forceinline__ void stream_rows(const SampleArgs& a, StreamKernelLds
       const uint32_t tid = opaque_tid();
       uint32_t pm = 0u;
       xm = 0u;
-      const bool last = (p + 1u) * kSPieceQ * 4u > V;  // the piece holds positions past V
+      const bool last = (p + 1u) * kSPieceQ * 4u > VL;  // the piece holds positions past VL
 #pragma unroll
       for (int c = 0; c < (int)kSNS; ++c) {
         const uint32_t i0 = 4u * (p * kSPieceQ + (uint32_t)c * kBlock + tid);
-        if (use_pen && i0 < V) pm |= ((L.hbits[(i0 >> 5) & (kSBits - 1u)] >> (i0 & 31u)) & 15u) << (4 * c);
+        if (use_pen && i0 < VL) pm |= ((L.hbits[(i0 >> 5) & (kSBits - 1u)] >> (i0 & 31u)) & 15u) << (4 * c);
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           const uint32_t i = i0 + (uint32_t)q;
-          if ((last && i >= V) || (masked && i < V && masked_out(a, i))) xm |= 1u << (4 * c + q);
+          if ((last && i >= VL) || (masked && i < VL && masked_out(a, i))) xm |= 1u << (4 * c + q);
         }
       }
       return pm;
@@ -378,9 +379,9 @@ __device__ __forceinline__ void stream_rows(const SampleArgs& a, StreamKernelLds
           list_piece(A, p, pmA, xmA);
           if (p == 0u) LLMHIP_MARK(10);
           if (p + 2u < np) {
-            stream_load<VEC>(A, row, V, p + 2u);
+            stream_load(A, row, VL, p + 2u);
           } else if (jn < nrows) {
-            stream_load<VEC>(A, a.logits + (size_t)bn * a.ld, V, 0u);
+            stream_load(A, a.logits + (size_t)bn * a.ld, VL, 0u);
             LLMHIP_MARK(9);
           }
           if (p == 0u) LLMHIP_MARK(11);
@@ -388,12 +389,27 @@ __device__ __forceinline__ void stream_rows(const SampleArgs& a, StreamKernelLds
           list_piece(Bf, p + 1u, pmB, xmB);
           if (p == 0u) LLMHIP_MARK(4);
           if (p + 3u < np) {
-            stream_load<VEC>(Bf, row, V, p + 3u);
+            stream_load(Bf, row, VL, p + 3u);
           } else if (jn < nrows) {
-            stream_load<VEC>(Bf, a.logits + (size_t)bn * a.ld, V, 1u);
+            stream_load(Bf, a.logits + (size_t)bn * a.ld, VL, 1u);
           }
         }
         fetched = true;
+        // The row's last V - VL values, one thread each.
+        if (TAIL && VL + tid < V) {
+          const uint32_t i = VL + tid;
+          const float v = ri.last;
+          if (v >= tf && !(masked && masked_out(a, i))) {
+            const uint64_t r = ((uint64_t)__float_as_uint(v) << 32) | i;
+            if (use_pen && ((L.hbits[(i >> 5) & (kSBits - 1u)] >> (i & 31u)) & 1u)) {
+              const uint32_t q = atomicAdd(&L.misc[kSPendN], 1u);
+              if (q < kSPend) L.pend[q] = r;
+            } else {
+              const uint32_t o = atomicAdd(&L.misc[kSCandN], 1u);
+              if (o < kSCand) L.list[o] = r;
+            }
+          }
+        }
         LLMHIP_MARK(5);
         lds_barrier();
         // The marked values' penalties (generate.rs:343-352), stopping once
@@ -471,8 +487,8 @@ __device__ __forceinline__ void stream_rows(const SampleArgs& a, StreamKernelLds
     // The next row's first two pieces, where not out yet (a row this path
     // did not list).
     if (!fetched) {
-      stream_load<VEC>(A, a.logits + (size_t)bn * a.ld, V, 0u);
-      stream_load<VEC>(Bf, a.logits + (size_t)bn * a.ld, V, 1u);
+      stream_load(A, a.logits + (size_t)bn * a.ld, VL, 0u);
+      stream_load(Bf, a.logits + (size_t)bn * a.ld, VL, 1u);
     }
     ri = ri_next;
     LLMHIP_MARK(8);

@@ -4,11 +4,11 @@
 
 namespace llmhip {
 
-template hipError_t launch_stream_k<false>(const SampleArgs&, bool, hipStream_t);
+template hipError_t launch_stream_k<false>(const SampleArgs&, hipStream_t);
 
 // bigk: some row of the launch has K > 64.
-hipError_t launch_stream(const SampleArgs& a, bool vec, bool bigk, hipStream_t s) {
-  return bigk ? launch_stream_k<true>(a, vec, s) : launch_stream_k<false>(a, vec, s);
+hipError_t launch_stream(const SampleArgs& a, bool bigk, hipStream_t s) {
+  return bigk ? launch_stream_k<true>(a, s) : launch_stream_k<false>(a, s);
 }
 
 }  // namespace llmhip
