@@ -145,11 +145,11 @@ int llmhip_sample_device(llmhip_ctx* ctx, const float* logits, size_t B, size_t 
  * :364). Same arguments, meaning and results as
  * llmhip_sample_device; the difference is where the device memory comes
  * from. This call allocates nothing: the per-row parameters (params_stride
- * != 0), the allowed mask's slot layout and the sorting path's per-row
+ * != 0) and the sorting path's per-row
  * scratch go into one array of LLMHIP_NOALLOC_SCRATCH_BYTES that the library
  * holds on each GPU it runs on, until the process ends. A call needs
  *   ceil(((B - 1) * params_stride + 1) * 20 / 256) * 256   (params, if per row)
- *   + 4096                                                 (mask layout)
+ *   + 4096                                                 (reserved)
  *   + B * w * Vp * 4                                       (scratch)
  * bytes, with Vp = V rounded up to 1024 and w = 2 when every row is greedy
  * or has 0 < top_k <= 4096, top_k < V, else 5. A larger call returns

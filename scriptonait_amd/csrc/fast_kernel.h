@@ -10,10 +10,10 @@ namespace llmhip {
 
 static_assert(kMaxFastK <= kSelCap, "hand-overs select in LDS");
 
-template <int NCH, bool GREEDY, bool CMODE, bool BIGK>
+template <int NCH, bool GREEDY, bool CMODE, bool BIGK, bool MASKED>
 __global__ __launch_bounds__(kBlock) void sample_fast_kernel(SampleArgs a) {
   __shared__ FastLds<NCH, BIGK> L;
-  if (__builtin_expect(!fast_row<NCH, GREEDY, CMODE, BIGK>(a, L), 0)) {
+  if (__builtin_expect(!fast_row<NCH, GREEDY, CMODE, BIGK, MASKED>(a, L), 0)) {
     if (threadIdx.x == 0) atomicAdd(a.handovers, 1u);
     __syncthreads();
     general_row<false>(a, launch_row(a), L.gen, true);  // greedy or K <= kMaxFastK: no whole-row sort
@@ -21,27 +21,33 @@ __global__ __launch_bounds__(kBlock) void sample_fast_kernel(SampleArgs a) {
 }
 
 // One launch per row class present: greedy rows and top-k rows run in
-// kernels compiled apart, so neither carries the other's registers. bigk:
-// some top-k row has K > 64.
-template <int NCH, bool CMODE>
-hipError_t launch_fast_nch(const SampleArgs& a0, bool bigk, hipStream_t s) {
+// kernels compiled apart, so neither carries the other's registers, and so do
+// calls with an allowed mask. bigk: some top-k row has K > 64.
+template <int NCH, bool CMODE, bool MASKED>
+hipError_t launch_fast_masked(const SampleArgs& a0, bool bigk, hipStream_t s) {
   SampleArgs a = a0;
   uint32_t grid;
   a.row_class_mask = kClassGreedy;
   if ((a0.row_class_mask & kClassGreedy) && (grid = launch_grid(a)) != 0u) {
-    hipLaunchKernelGGL((sample_fast_kernel<NCH, true, CMODE, false>), dim3(grid), dim3(kBlock), 0, s, a);
+    hipLaunchKernelGGL((sample_fast_kernel<NCH, true, CMODE, false, MASKED>), dim3(grid), dim3(kBlock), 0, s, a);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
   a.row_class_mask = kClassTopK;
   if ((a0.row_class_mask & kClassTopK) && (grid = launch_grid(a)) != 0u) {
     if (bigk) {
-      hipLaunchKernelGGL((sample_fast_kernel<NCH, false, CMODE, true>), dim3(grid), dim3(kBlock), 0, s, a);
+      hipLaunchKernelGGL((sample_fast_kernel<NCH, false, CMODE, true, MASKED>), dim3(grid), dim3(kBlock), 0, s, a);
     } else {
-      hipLaunchKernelGGL((sample_fast_kernel<NCH, false, CMODE, false>), dim3(grid), dim3(kBlock), 0, s, a);
+      hipLaunchKernelGGL((sample_fast_kernel<NCH, false, CMODE, false, MASKED>), dim3(grid), dim3(kBlock), 0, s, a);
     }
   }
   return hipGetLastError();
+}
+
+template <int NCH, bool CMODE>
+hipError_t launch_fast_nch(const SampleArgs& a, bool bigk, hipStream_t s) {
+  return a.allowed || a.allowed_bits ? launch_fast_masked<NCH, CMODE, true>(a, bigk, s)
+                                     : launch_fast_masked<NCH, CMODE, false>(a, bigk, s);
 }
 
 // Each (NCH, CMODE) instantiation is compiled in a file of its own

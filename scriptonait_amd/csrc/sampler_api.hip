@@ -15,9 +15,8 @@
 // Device memory of llmhip_sample_device_noalloc, for callers that cannot
 // allocate: each GPU the library runs on holds its own copy of this array
 // until the process ends. One call lays out, from the start: the per-row
-// parameters (when params_stride != 0), the allowed mask in the register
-// path's slot layout (kBlock words), and the per-row scratch of the sorting
-// path. Host code never passes `scratch` itself to a kernel or a copy (in
+// parameters (when params_stride != 0), kBlock reserved words, and the per-row
+// scratch of the sorting path. Host code never passes `scratch` itself to a kernel or a copy (in
 // host code the name is a host-side stand-in, not a device address): it uses
 // the address hipGetSymbolAddress returns for the current device, looked up
 // once per device when the first context on that device is created.
@@ -28,7 +27,6 @@ hipError_t launch_fast(const SampleArgs& a, bool bigk, hipStream_t s);
 hipError_t launch_fast_counts(const SampleArgs& a, bool bigk, hipStream_t s);
 hipError_t launch_general(const SampleArgs& a, hipStream_t s);
 hipError_t launch_vocab(const SampleArgs& a, bool plain, hipStream_t s);
-hipError_t launch_slotmask(const SampleArgs& a, uint32_t* out, hipStream_t s);
 hipError_t launch_seen_bits(const uint32_t* tokens, uint64_t n, uint32_t V, uint32_t* bits, hipStream_t s);
 hipError_t launch_take_status(uint32_t* words, hipStream_t s);
 hipError_t launch_stream(const SampleArgs& a, bool bigk, hipStream_t s);
@@ -106,8 +104,6 @@ struct llmhip_ctx {
   hipStream_t stream = nullptr;  // used by the host entry
   DevBuf scratch;                // general-path per-row scratch
   DevBuf params;                 // per-row params copied from the host
-  DevBuf zeros;                  // kBlock zero words: the fast path's "no mask" slot mask
-  DevBuf slotmask;               // kBlock words: the allowed mask in the fast path's layout
   DevBuf status;                 // kStatusWords words: kernel flags (host / device calls) and the hand-over count
   DevBuf head_logits;            // the tied head's logits when the caller does not take them
   uint32_t spin_limit = kSpinLimit;  // bound of the kernels' waits between wavefronts
@@ -189,7 +185,6 @@ struct Mask {
 struct Workspace {
   uint32_t* scratch = nullptr;  // per-row scratch, scratch_bytes long
   size_t scratch_bytes = 0;
-  uint32_t* slotmask = nullptr;  // kBlock words
 };
 
 // Scratch words per row that a call may touch (row_scratch_words over its
@@ -288,7 +283,6 @@ int enqueue(llmhip_ctx* ctx, const float* logits, size_t B, size_t V, size_t ld,
   a.out_ids = out_ids;
   a.out_probs = out_probs;
   a.out_kept = out_kept;
-  a.slotmask = static_cast<const uint32_t*>(ctx->zeros.ptr);
   a.status = static_cast<uint32_t*>(ctx->status.ptr) + (host_call ? kStatusHostWord : kStatusDeviceWord);
   a.handovers = static_cast<uint32_t*>(ctx->status.ptr) + kStatusHandoverWord;
   a.spin_limit = ctx->spin_limit;
@@ -304,15 +298,6 @@ int enqueue(llmhip_ctx* ctx, const float* logits, size_t B, size_t V, size_t ld,
 
   if (out_probs) HIP_TRY(hipMemsetAsync(out_probs, 0, B * V * sizeof(float), s));
   if (fast_mask) {
-    if (a.allowed || a.allowed_bits) {
-      uint32_t* sm = ws ? ws->slotmask : nullptr;
-      if (!sm) {
-        if ((st = ctx->slotmask.ensure(kBlock * sizeof(uint32_t)))) return st;
-        sm = static_cast<uint32_t*>(ctx->slotmask.ptr);
-      }
-      HIP_TRY(launch_slotmask(a, sm, s));
-      a.slotmask = sm;
-    }
     a.row_class_mask = fast_mask;
     HIP_TRY(a.counts ? launch_fast_counts(a, bigk, s) : launch_fast(a, bigk, s));
   }
@@ -433,15 +418,12 @@ int llmhip_ctx_create(int device, llmhip_ctx** out_ctx) {
     delete ctx;
     return hip_fail(e, "hipStreamCreateWithFlags");
   }
-  int st = ctx->zeros.ensure(kBlock * sizeof(uint32_t));
-  if (st == LLMHIP_OK) st = ctx->status.ensure(kStatusWords * sizeof(uint32_t));
+  int st = ctx->status.ensure(kStatusWords * sizeof(uint32_t));
   if (st == LLMHIP_OK) {
-    e = hipMemset(ctx->zeros.ptr, 0, kBlock * sizeof(uint32_t));
-    if (e == hipSuccess) e = hipMemset(ctx->status.ptr, 0, kStatusWords * sizeof(uint32_t));
+    e = hipMemset(ctx->status.ptr, 0, kStatusWords * sizeof(uint32_t));
     if (e != hipSuccess) st = hip_fail(e, "hipMemset");
   }
   if (st != LLMHIP_OK) {
-    ctx->zeros.release();
     ctx->status.release();
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
@@ -456,7 +438,7 @@ int llmhip_ctx_destroy(llmhip_ctx* ctx) {
   Device d(ctx->device);
   if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
   (void)hipDeviceSynchronize();
-  for (DevBuf* b : {&ctx->scratch, &ctx->params, &ctx->zeros, &ctx->slotmask, &ctx->status, &ctx->head_logits,
+  for (DevBuf* b : {&ctx->scratch, &ctx->params, &ctx->status, &ctx->head_logits,
                     &ctx->logits, &ctx->hist, &ctx->hoff, &ctx->allowed, &ctx->rng, &ctx->ids, &ctx->probs, &ctx->kept})
     b->release();
   if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
@@ -504,7 +486,7 @@ int llmhip_sample_device_noalloc(llmhip_ctx* ctx, const float* logits, size_t B,
                        : std::string("no-alloc scratch: no device address for this device");
     return LLMHIP_ERR_HIP;
   }
-  // The call's layout in the array: params | slot mask | per-row scratch.
+  // The call's layout in the array: params | reserved | per-row scratch.
   const size_t pbytes =
       params_stride ? (((B - 1) * params_stride + 1) * sizeof(llmhip_params) + 255u) / 256u * 256u : 0u;
   const size_t mbytes = kBlock * sizeof(uint32_t);
@@ -527,7 +509,6 @@ int llmhip_sample_device_noalloc(llmhip_ctx* ctx, const float* logits, size_t B,
     pdev = reinterpret_cast<const llmhip_params*>(base);
   }
   Workspace ws;
-  ws.slotmask = reinterpret_cast<uint32_t*>(base + pbytes);
   ws.scratch = reinterpret_cast<uint32_t*>(base + pbytes + mbytes);
   ws.scratch_bytes = (size_t)LLMHIP_NOALLOC_SCRATCH_BYTES - pbytes - mbytes;
   Mask m;

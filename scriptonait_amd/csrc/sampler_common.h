@@ -60,10 +60,6 @@ struct SampleArgs {
   const uint8_t* allowed;        // device, may be null
   const uint32_t* allowed_bits;  // device, may be null
   uint32_t allowed_len;
-  // Fast path: bit e of word t is set when thread t's slot e is masked out
-  // by the allowed mask (the fast kernel's layout, built by a prep kernel),
-  // or all zeros when there is no mask. 1024 words, always valid.
-  const uint32_t* slotmask;
   // Decode-step mode (ring_cap > 0): row b's history is the last
   // min(ring_len[b] - hist_start[b], window) tokens of the ring ring[b*ring_cap
   // .. (b+1)*ring_cap) (hist == ring, hist_offsets == null); each result is

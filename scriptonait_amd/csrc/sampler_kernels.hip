@@ -43,26 +43,6 @@ __global__ __launch_bounds__(kBlock) void sample_general_kernel(SampleArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// Allowed mask in the fast kernel's slot layout: word t, bit 4c+j is set when
-// the position of thread t's chunk c, float j is masked out
-// (generate.rs:333-341). One workgroup; built once per call, shared by all
-// rows.
-// ---------------------------------------------------------------------------
-template <int NCH>
-__global__ __launch_bounds__(kBlock) void slotmask_kernel(SampleArgs a, uint32_t* out) {
-  const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63u;
-  uint32_t m = 0u;
-  for (int c = 0; c < NCH; ++c) {
-    const uint32_t base = chunk_pos<NCH>((uint32_t)c, wave, lane);
-    for (int j = 0; j < 4; ++j) {
-      const uint32_t p = base + j;
-      if (p < a.V && masked_out(a, p)) m |= 1u << (4 * c + j);
-    }
-  }
-  out[tid] = m;
-}
-
-// ---------------------------------------------------------------------------
 // Allowed mask as bits from a corpus's tokens (Corpus::seen_tokens,
 // crates/llm-core/src/corpus.rs:236-247): bit id is set when some token
 // equals id < V; larger ids are ignored, as seen.get_mut(id) ignores them.
@@ -105,16 +85,6 @@ __global__ __launch_bounds__(kBlock) void seen_bits_kernel(const uint32_t* token
 // ---------------------------------------------------------------------------
 // Host-side launch.
 // ---------------------------------------------------------------------------
-hipError_t launch_slotmask(const SampleArgs& a, uint32_t* out, hipStream_t s) {
-  switch (fast_nch(a.V)) {
-    case 1: hipLaunchKernelGGL(slotmask_kernel<1>, dim3(1), dim3(kBlock), 0, s, a, out); break;
-    case 2: hipLaunchKernelGGL(slotmask_kernel<2>, dim3(1), dim3(kBlock), 0, s, a, out); break;
-    case 4: hipLaunchKernelGGL(slotmask_kernel<4>, dim3(1), dim3(kBlock), 0, s, a, out); break;
-    default: hipLaunchKernelGGL(slotmask_kernel<8>, dim3(1), dim3(kBlock), 0, s, a, out); break;
-  }
-  return hipGetLastError();
-}
-
 // Calls without a count table (decode steps with one: fast_counts.hip).
 hipError_t launch_fast(const SampleArgs& a, bool bigk, hipStream_t s) {
   return launch_fast_mode<false>(a, bigk, s);
