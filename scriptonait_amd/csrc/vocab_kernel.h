@@ -18,8 +18,7 @@ __global__ __launch_bounds__(kBlock) void sample_vocab_kernel(SampleArgs a) {
   const uint32_t b = launch_row(a);
   if (b >= a.B) return;
   if (!a.row_cls_on && !(route_class(load_params(a, b), a.V) & a.row_class_mask)) return;
-  const bool vec4 = (reinterpret_cast<uintptr_t>(a.logits) % 16u == 0u) && (a.ld % 4u == 0u);
-  if (!vocab_row<PLAIN>(a, b, L.v, vec4)) {
+  if (!vocab_row<PLAIN>(a, b, L.v, a.V >= 4u)) {
     if (threadIdx.x == 0) atomicAdd(a.handovers, 1u);
     __syncthreads();
     general_row(a, b, L.gen, true);

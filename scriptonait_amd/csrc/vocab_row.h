@@ -193,7 +193,7 @@ __device__ __forceinline__ double block_scan_f64(double x, double* tmp, double& 
 // row, w being the masked, penalized logit divided by the temperature.
 // Row streamed from memory by every pass: float4 groups, two batches of 4
 // per thread in flight (the next batch loads while this one is visited), or
-// scalars when the row is not 16-byte aligned.
+// scalars when the row has fewer than four values (vec4 false).
 //
 // VP gives an element's value in parts: pre(i, v) the allowed mask, pen()
 // whether the row has penalized history ids, hit(i) / hit4(i) their filter
@@ -208,6 +208,16 @@ struct StreamSrc {
   uint32_t V;
   bool vec4;
   VP vp;
+  // Floats 4q .. 4q+3 of the row, q below its V / 4 whole quads (zeros past
+  // them). Rows need no alignment beyond a float's: gfx950's 16-byte global
+  // loads take any 4-byte aligned address (256 rows of 32001: 224.5 -> 216.3 us
+  // against a load per value).
+  __device__ __forceinline__ float4 quad(uint32_t q, uint32_t nq) const {
+    typedef float f4v __attribute__((ext_vector_type(4), aligned(4)));
+    if (q >= nq) return make_float4(0.f, 0.f, 0.f, 0.f);
+    const f4v v = *reinterpret_cast<const f4v*>(row + 4u * q);
+    return make_float4(v.x, v.y, v.z, v.w);
+  }
   // Element i's value from its logit v.
   __device__ __forceinline__ float value(uint32_t i, float v) const {
     v = vp.pre(i, v);
@@ -233,10 +243,10 @@ struct StreamSrc {
     for (int q = 0; q < 16; ++q)
       if ((valid >> q) & 1u) w[q] = vp.post(w[q]);
   }
-  // Elements 4 * (q0 + t + kBlock * s) + c of float4 groups cur[s], s < 4:
-  // their pre() values, validity and history marks.
-  __device__ __forceinline__ void pre_quads(const float4 (&v4)[4], uint32_t base, uint32_t stride, float (&w)[16],
-                                            uint32_t& valid, uint32_t& hm) const {
+  // Elements 4 * (base + stride * s) + c of float4 groups v4[s], s < 4: their
+  // pre() values, validity (those below end) and history marks.
+  __device__ __forceinline__ void pre_quads(const float4 (&v4)[4], uint32_t base, uint32_t stride, uint32_t end,
+                                            float (&w)[16], uint32_t& valid, uint32_t& hm) const {
     valid = 0u;
     hm = 0u;
 #pragma unroll
@@ -246,11 +256,19 @@ struct StreamSrc {
       const uint32_t hb = vp.pen() ? vp.hit4(i) : 0u;  // one filter word holds the four ids
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
-        const bool in = i + c < V;
+        const bool in = i + c < end;
         w[4 * s + c] = in ? vp.pre(i + c, v[c]) : 0.0f;
         valid |= (in ? 1u : 0u) << (4 * s + c);
         hm |= (in && ((hb >> c) & 1u) ? 1u : 0u) << (4 * s + c);
       }
+    }
+  }
+  // The row's last V % 4 values, one thread each.
+  template <class F>
+  __device__ __forceinline__ void last_few(F&& f) const {
+    if ((V & 3u) != 0u) {
+      const uint32_t i = (V & ~3u) + threadIdx.x;
+      if (i < V) f(value_at(i), i);
     }
   }
   template <class F>
@@ -260,19 +278,18 @@ struct StreamSrc {
     if (!vp.pen()) {
       // No history ids: each element's value as it is visited.
       if (vec4) {
-        const float4* r4 = reinterpret_cast<const float4*>(row);
-        const uint32_t nq = (V + 3u) / 4u;
+        const uint32_t nq = V / 4u;
         float4 cur[4], nxt[4];
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
           const uint32_t q = t + nt * s;
-          cur[s] = q < nq ? r4[q] : make_float4(0.f, 0.f, 0.f, 0.f);
+          cur[s] = quad(q, nq);
         }
         for (uint32_t q0 = 0; q0 < nq; q0 += 4u * nt) {
 #pragma unroll
           for (int s = 0; s < 4; ++s) {
             const uint32_t q = q0 + 4u * nt + t + nt * s;
-            nxt[s] = q < nq ? r4[q] : make_float4(0.f, 0.f, 0.f, 0.f);
+            nxt[s] = quad(q, nq);
           }
 #pragma unroll
           for (int s = 0; s < 4; ++s) {
@@ -280,11 +297,12 @@ struct StreamSrc {
             const float v[4] = {cur[s].x, cur[s].y, cur[s].z, cur[s].w};
 #pragma unroll
             for (int c = 0; c < 4; ++c)
-              if (i + c < V) f(vp.post(vp.pre(i + c, v[c])), i + c);
+              if (i < (V & ~3u)) f(vp.post(vp.pre(i + c, v[c])), i + c);
           }
 #pragma unroll
           for (int s = 0; s < 4; ++s) cur[s] = nxt[s];
         }
+        last_few(f);
       } else {
         uint32_t i = t;
         for (; i + 7u * nt < V; i += 8u * nt) {
@@ -301,21 +319,20 @@ struct StreamSrc {
     float w[16];
     uint32_t valid, hm;
     if (vec4) {
-      const float4* r4 = reinterpret_cast<const float4*>(row);
-      const uint32_t nq = (V + 3u) / 4u;
+      const uint32_t nq = V / 4u;
       float4 cur[4], nxt[4];
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
         const uint32_t q = t + nt * s;
-        cur[s] = q < nq ? r4[q] : make_float4(0.f, 0.f, 0.f, 0.f);
+        cur[s] = quad(q, nq);
       }
       for (uint32_t q0 = 0; q0 < nq; q0 += 4u * nt) {
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
           const uint32_t q = q0 + 4u * nt + t + nt * s;
-          nxt[s] = q < nq ? r4[q] : make_float4(0.f, 0.f, 0.f, 0.f);
+          nxt[s] = quad(q, nq);
         }
-        pre_quads(cur, q0 + t, nt, w, valid, hm);
+        pre_quads(cur, q0 + t, nt, V & ~3u, w, valid, hm);
         finish(w, valid, hm, [&](uint32_t e) { return 4u * (q0 + t + nt * (e >> 2)) + (e & 3u); });
 #pragma unroll
         for (int e = 0; e < 16; ++e)
@@ -323,6 +340,7 @@ struct StreamSrc {
 #pragma unroll
         for (int s = 0; s < 4; ++s) cur[s] = nxt[s];
       }
+      last_few(f);
     } else {
       for (uint32_t i0 = t; i0 < V; i0 += 16u * nt) {
 #pragma unroll
@@ -358,13 +376,17 @@ struct StreamSrc {
     const uint32_t lane = threadIdx.x & 63u;
     uint32_t hm;
     if (vec4) {
-      const float4* r4 = reinterpret_cast<const float4*>(row);
-      const uint32_t nq = (V + 3u) / 4u;
+      const uint32_t nq = V / 4u;
       float4 v4[4];
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
         const uint32_t q = blk * 256u + lane + 64u * s;
-        v4[s] = q < nq ? r4[q] : make_float4(0.f, 0.f, 0.f, 0.f);
+        v4[s] = quad(q, nq);
+        if ((V & 3u) != 0u && q == nq) {  // the row's last few
+          v4[s].x = row[4u * q];
+          if ((V & 3u) > 1u) v4[s].y = row[4u * q + 1u];
+          if ((V & 3u) > 2u) v4[s].z = row[4u * q + 2u];
+        }
       }
 #pragma unroll
       for (int e = 0; e < 16; ++e) id[e] = 4u * (blk * 256u + lane + 64u * (uint32_t)(e >> 2)) + (uint32_t)(e & 3);
@@ -382,7 +404,7 @@ struct StreamSrc {
         }
         return;
       }
-      pre_quads(v4, blk * 256u + lane, 64u, w, valid, hm);
+      pre_quads(v4, blk * 256u + lane, 64u, V, w, valid, hm);
       finish(w, valid, hm, [&](uint32_t e) { return 4u * (blk * 256u + lane + 64u * (e >> 2)) + (e & 3u); });
     } else {
 #pragma unroll
@@ -438,18 +460,26 @@ struct ListSrc {
   }
 };
 
-// exp(y) for -80 <= y <= 0 from the hardware exp2: y * log2(e) = k + f with
-// the product split exactly by an FMA, |f| <= 1/2, and v_exp_f32, whose
-// relative error on [-1/2, 1/2] is at most 1.4 * 2^-24 (measured over every
-// input). The result is within 2^-22 of glibc's expf (which is itself within
-// 0.502 ulp of exp). Used only to settle decisions that have that much room.
-__device__ __forceinline__ float cheap_x(float y) {
-  const float L1 = 0x1.715476p+0f, L2 = 0x1.4ae0bep-26f;  // log2(e) = L1 + L2 + O(2^-50)
-  const float hi = y * L1;
-  const float lo = __builtin_fmaf(y, L1, -hi) + y * L2;
-  const float kf = rintf(hi);
-  const float f = (hi - kf) + lo;  // hi - kf is exact
-  return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(f), (int)kf);
+// glibc_expf_tab's steps for kExactMin <= y <= 0, without its tests for the
+// ends of the range: the same value, in binary64 (which gfx950 runs at the
+// vector ALU's binary32 rate).
+constexpr float kExactMin = -60.0f;
+__device__ __forceinline__ float exact_x(float y, const uint64_t* tab) {
+  const double kInvLn2N = 0x1.71547652b82fep+0 * 32.0;
+  const double kShift = 0x1.8p+52;
+  const double kC0 = 0x1.c6af84b912394p-5 / (32.0 * 32.0 * 32.0);
+  const double kC1 = 0x1.ebfce50fac4f3p-3 / (32.0 * 32.0);
+  const double kC2 = 0x1.62e42ff0c52d6p-1 / 32.0;
+  const double yd = (double)y;
+  double kd = __builtin_fma(kInvLn2N, yd, kShift);
+  const uint32_t ki = (uint32_t)f64_bits(kd);
+  kd -= kShift;
+  const double r = __builtin_fma(kInvLn2N, yd, -kd);
+  const uint64_t e = tab[ki % 32u];  // + ki << 47, which reaches the upper word only
+  const double s = f64_from_bits(((uint64_t)((uint32_t)(e >> 32) + (ki << 15)) << 32) | (uint32_t)e);
+  const double z = __builtin_fma(kC0, r, kC1);
+  const double p = __builtin_fma(z, r * r, __builtin_fma(kC2, r, 1.0));
+  return (float)(p * s);
 }
 
 // One or two folds over the row's terms in sorted order (see the file
@@ -687,37 +717,34 @@ __device__ __forceinline__ bool run_folds(FoldSpec (&fs)[NF], float mx, float u,
   __syncthreads();
 
   // Exact pass: certain buckets add ulp counts, zones gather, ties are listed.
-  // A term is first taken from a cheap exp (cheap_x: within 2^-22 of glibc's
-  // expf, and after the reciprocal multiply within 2^-20 of the exact term);
-  // the exact term is computed only when the cheap one cannot settle the
-  // min-p test or an ulp count (a scaled value within value * 2^-20 of a
-  // half-integer, or a term near the binade).
-  const float rcpS = S > 0.0f ? 1.0f / S : 1.0f;
+  // Every term is the exact one: x in binary64 as glibc's expf computes it,
+  // and x / S as x * (1 / S) in binary64, rounded once. (The binary64 product
+  // is within 2^-52 of the quotient of two 24-bit significands, and no such
+  // quotient lies within 2^-49 of a midpoint of two binary32 values: it would
+  // be a ratio whose numerator a 25-bit odd factor divides. kExactMin keeps
+  // the quotient a normal number.)
+  // The pass is bound by issue. Taking a term from the hardware exp2, and the
+  // exact one only where that could not settle the count (1.6% of the
+  // elements, but two wave positions in three), was longer: 1024 rows of 50257
+  // with top_p 0.98 took 1025 us, and 946 so. Not kept: the 16 elements of a
+  // thread in one branch-free stretch, two or four at a time, with the zone
+  // elements and ties taken one by one behind it (989-1095 us).
+  const double rcpS = S > 0.0f ? 1.0 / (double)S : 1.0;
   uint32_t nin = 0;
   src.for_each([&](float w, uint32_t i) __attribute__((always_inline)) {
     const float y = w - mx;
     const uint32_t k = vbucket(y);
     const uint32_t bi = L.binfo[k];
-    // The cheap term is computed while the bucket's word is read (the
-    // empty asm keeps it ahead of the class test that waits for the read).
-    const bool cheap = y >= -80.0f;
-    float ta = cheap ? cheap_x(y) * rcpS : 0.0f;
-    asm volatile("" : "+v"(ta));
+    float t;
+    if (__builtin_expect(y >= kExactMin, 1)) {
+      t = exact_x(y, L.exptab);
+      if constexpr (NF == 2) t = (float)((double)t * rcpS);
+    } else {
+      t = term_of(glibc_expf_tab(y, L.exptab));
+    }
     const uint32_t c0 = bcls(bi, 0), c1 = bcls(bi, 1);
     if (c0 == kBSkip && c1 == kBSkip) return;
-    float t = -1.0f;  // the exact term, once computed
-    if (thr > 0.0f) {
-      bool in;
-      if (cheap && ta >= thr * (1.0f + 0x1p-19f)) {
-        in = true;
-      } else if (cheap && ta < thr * (1.0f - 0x1p-19f)) {
-        in = false;
-      } else {
-        t = term_of(glibc_expf_tab(y, L.exptab));
-        in = t >= thr;
-      }
-      if (!in) return;
-    }
+    if (thr > 0.0f && !(t >= thr)) return;
     if (c0 != kBSkip) ++nin;
     // A gathered bucket that is certain for the other fold is also counted
     // for it, so that fold adds it as one integer.
@@ -731,36 +758,26 @@ __device__ __forceinline__ bool run_folds(FoldSpec (&fs)[NF], float mx, float u,
 #pragma unroll
     for (int f = 0; f < NF; ++f) {
       if ((f == 0 ? c0 : c1) != kBCert) continue;
-      const int E = bbin(bi, f);
-      if (cheap && t < 0.0f) {
-        const float v = __builtin_amdgcn_ldexpf(ta, 23 - E);  // ta in units of 2^(E-23), exactly
-        if (v < 0x1p22f) {
-          const float fl = floorf(v), fr = v - fl;
-          if (fabsf(fr - 0.5f) > v * 0x1p-20f + 0x1p-40f) {
-            atomicAdd(&Df(f)[k], (uint32_t)fl + (fr > 0.5f ? 1u : 0u));
-            continue;
+      // t in units of 2^(E-23): exact (or, where it underflows, below 1/2).
+      const float v = __builtin_amdgcn_ldexpf(t, 23 - bbin(bi, f));
+      const bool big = v >= 0x1p23f, tie = __builtin_amdgcn_fractf(v) == 0.5f;
+      if (__builtin_expect(big || tie, 0)) {
+        if (gath) {
+          atomicOr(&L.binfo[k], kBStep << f);  // this fold replays the bucket element by element
+        } else if (big) {
+          L.misc[kVFail] = 1u;  // (a certain bucket never holds such a term)
+        } else {
+          const uint32_t s = atomicAdd(&L.misc[kVNTies], 1u);
+          if (s < kVTies) {
+            L.tkey[s] = f2key(w);
+            L.tidx[s] = i;
+            L.tq[s] = (uint32_t)floorf(v);
+            L.tbk[s] = k | ((uint32_t)f << 31);
+            L.tab[s] = 0u;
           }
         }
-      }
-      if (t < 0.0f) t = term_of(glibc_expf_tab(y, L.exptab));
-      bool tie, big;
-      const uint32_t q = rne_units(t, E, tie, big);
-      if (gath && (tie || big)) {
-        atomicOr(&L.binfo[k], kBStep << f);  // this fold replays the bucket element by element
-        continue;
-      }
-      if (big) L.misc[kVFail] = 1u;
-      if (tie) {
-        const uint32_t s = atomicAdd(&L.misc[kVNTies], 1u);
-        if (s < kVTies) {
-          L.tkey[s] = f2key(w);
-          L.tidx[s] = i;
-          L.tq[s] = q;
-          L.tbk[s] = k | ((uint32_t)f << 31);
-          L.tab[s] = 0u;
-        }
       } else {
-        atomicAdd(&Df(f)[k], q);
+        atomicAdd(&Df(f)[k], (uint32_t)__builtin_rintf(v));
       }
     }
   });

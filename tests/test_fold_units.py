@@ -146,3 +146,40 @@ def test_a_subtraction_that_lands_on_the_binade_floor_can_round_below_it():
     assert (ref == (np.ldexp(1.0, E) - u / 2).astype(np.float32)).all()  # ... f32 rounds below it
     inside, _, _ = _check(F, t, sub=True)
     assert not inside.any()
+
+
+DIV = textwrap.dedent(r"""
+    #include <stdint.h>
+    #include <stdio.h>
+    #include <string.h>
+    static uint64_t s = 1;
+    static uint32_t rnd(void) { s = s * 6364136223846793005ull + 1442695040888963407ull; return (uint32_t)(s >> 32); }
+    static float bits(uint32_t u) { float f; memcpy(&f, &u, 4); return f; }
+    int main(void) {
+      unsigned long bad = 0;
+      for (long i = 0; i < 60000000; ++i) {
+        /* S in [1, 2^31), x in [2^-87, 1]: significands random, or a few ulps from a power of two */
+        uint32_t mx = rnd() & 0x7fffff, ms = rnd() & 0x7fffff;
+        if (i & 1) mx = (rnd() & 7) * ((rnd() & 1) ? 1u : 0x7fffffu) & 0x7fffff;
+        if (i & 2) ms = (rnd() & 7) * ((rnd() & 1) ? 1u : 0x7fffffu) & 0x7fffff;
+        volatile float S = bits((127 + rnd() % 31) << 23 | ms), x = bits((127 - rnd() % 87) << 23 | mx);
+        volatile double r = 1.0 / (double)S;
+        volatile float q = x / S, p = (float)((double)x * r);
+        if (q != p) ++bad;
+      }
+      printf("%lu\n", bad);
+      return 0;
+    }
+""")
+
+
+def test_a_quotient_is_its_binary64_reciprocal_product_rounded_once(tmp_path):
+    """x / S in binary32 equals x * (1 / S) in binary64 rounded to binary32
+    for the folds' terms: the product is within 2^-52 of the quotient, and a
+    quotient of two 24-bit significands is never within 2^-49 of a midpoint."""
+    src = tmp_path / "div.c"
+    src.write_text(DIV)
+    exe = tmp_path / "div"
+    subprocess.run(["gcc", "-O2", "-ffp-contract=off", str(src), "-o", str(exe)], check=True)
+    out = subprocess.run([str(exe)], check=True, capture_output=True, text=True, timeout=120).stdout
+    assert int(out) == 0

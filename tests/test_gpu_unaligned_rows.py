@@ -1,6 +1,6 @@
 """GPU: rows that start at any float (odd strides, an offset base), whose
-length is not a multiple of 4: the register, greedy and streaming kernels'
-16-byte loads against the oracle.
+length is not a multiple of 4: the register, greedy, streaming and
+full-vocabulary kernels' 16-byte loads against the oracle.
 
 Each row's largest values include its first and its last ones, so a value
 lost or moved at either end changes the ids."""
@@ -16,7 +16,7 @@ pytestmark = pytest.mark.gpu
 def _params(B):
     prm = np.zeros(B, dtype=PARAMS_DTYPE)
     prm["temperature"] = np.where(np.arange(B) % 3 == 2, 0.0, 0.8)
-    prm["top_k"] = np.where(np.arange(B) % 2 == 0, 3, 100)
+    prm["top_k"] = np.where(np.arange(B) % 2 == 0, 3, np.where(np.arange(B) == 3, 0, 100))
     prm["top_p"] = 0.95
     prm["min_p"] = 0.0
     prm["repetition_penalty"] = 1.2
