@@ -222,14 +222,14 @@ int enqueue(llmhip_ctx* ctx, const float* logits, size_t B, size_t V, size_t ld,
     return LLMHIP_OK;
   }
   uint32_t classes = 0;
-  bool bigk = false;  // some top-k row of the register path has K > 64
+  bool bigk = false;  // some top-k row has K > 64, or more to list than the small-K kernels rank
   bool penalized = false;  // some row has a repetition penalty (and the call a history)
   uint32_t row_cls[128] = {};  // each row's class index (SampleArgs::row_cls), for calls of <= kRowClsRows rows
   for (size_t b = 0; b < (params_stride ? B : 1); ++b) {
     const llmhip_params& p = params_host[b * params_stride];
     const uint32_t c = route_class(p, (uint32_t)V);
     classes |= c;
-    bigk = bigk || (c == kClassTopK && p.top_k > 64u);
+    bigk = bigk || (c == kClassTopK && (p.top_k > 64u || (V > kMaxFastV && stream_bigk(p.top_k, (uint32_t)V))));
     penalized = penalized || p.repetition_penalty != 1.0f;
     if (b < kRowClsRows) row_cls[b >> 4] |= (uint32_t)__builtin_ctz(c) << ((b & 15u) * 2u);
   }

@@ -366,14 +366,34 @@ __host__ __device__ __forceinline__ uint32_t row_class(const llmhip_params& p, u
 
 // The streaming path (top-k rows past kMaxFastV) lists about 1.2 K values
 // per 32768 of the row (its threshold comes from the row's first 32768
-// values) in a list of kStreamCand: it takes a row when that fits with a
-// margin, and when the penalty is at least 1 (one below 1 can raise a value
-// past the threshold).
+// values) in a list of kStreamCand. Where that does not fit with a margin, or
+// K is above 256, it raises the threshold after each 32768 values: part j then
+// lists about K / j, and the first at most 1.45 K (the first threshold is the
+// lower edge of a bin 1/8 of a value wide). It takes a row when either fits,
+// and when the penalty is at least 1 (one below 1 can raise a value past the
+// threshold).
 constexpr uint32_t kStreamSpan = 32768;
 constexpr uint32_t kStreamCand = 4096;
+__host__ __device__ __forceinline__ uint32_t stream_parts(uint32_t V) { return (V + kStreamSpan - 1u) / kStreamSpan; }
+__host__ __device__ __forceinline__ bool stream_fits(uint32_t K, uint32_t V) {
+  return (uint64_t)K * stream_parts(V) * 5u <= (uint64_t)kStreamCand * 4u;
+}
+__host__ __device__ __forceinline__ bool stream_refines(uint32_t K, uint32_t V) {
+  return K > 256u || !stream_fits(K, V);
+}
+// Rows of K <= 64 that the streaming kernel compiled for them may hand over
+// (it ranks 512 listed values, of about 1.25 K per part).
+__host__ __device__ __forceinline__ bool stream_bigk(uint32_t K, uint32_t V) {
+  return stream_refines(K, V) || (uint64_t)K * stream_parts(V) * 3u > 1024u;
+}
 __host__ __device__ __forceinline__ bool stream_takes(const llmhip_params& p, uint32_t V) {
-  const uint32_t parts = (V + kStreamSpan - 1u) / kStreamSpan;
-  return (uint64_t)p.top_k * parts * 5u <= (uint64_t)kStreamCand * 4u && p.repetition_penalty >= 1.0f;
+  if (!(p.repetition_penalty >= 1.0f)) return false;
+  if (stream_fits(p.top_k, V)) return true;
+  // 1 + 1/2 + ... + 1/(parts - 1) is at most 1 + 5/6 (m - 1), m the bit length
+  // of parts - 1 (V > kMaxFastV: at least two parts); 15/16 of the list.
+  uint32_t m = 0u;
+  for (uint32_t n = stream_parts(V) - 1u; n != 0u; n >>= 1) ++m;
+  return (uint64_t)p.top_k * (147u + 50u * (m - 1u)) <= (uint64_t)kStreamCand * 15u / 16u * 60u;
 }
 
 // The path a row is routed to: its class, except that a top-k row past the

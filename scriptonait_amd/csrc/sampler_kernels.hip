@@ -38,7 +38,7 @@ __global__ __launch_bounds__(kBlock) void sample_general_kernel(SampleArgs a) {
   __shared__ GenLds L;
   const uint32_t b = launch_row(a);
   if (b >= a.B) return;
-  if (!a.row_cls_on && !(route_class(load_params(a, b), a.V) & a.row_class_mask)) return;
+  if (a.params && !a.row_cls_on && !(route_class(load_params(a, b), a.V) & a.row_class_mask)) return;
   general_row(a, b, L, false);
 }
 

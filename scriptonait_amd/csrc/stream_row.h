@@ -32,6 +32,14 @@
 //     folds and the draw (draw_tail_bcast for K <= 64, draw_tail_lds
 //     above), while the other waves issue the next row's loads.
 //
+// Rows of a large K raise the threshold after every two pieces: a histogram
+// of the unmarked values listed so far, in bins of 1/512 of a value, gives
+// their K-th largest, and the row's last one cuts the list to little more than
+// K before the sort. (From the first threshold alone a row lists 1.2-1.4 K
+// values per 32768, so 512 rows of 131072 at top_k 1000 did not fit the list
+// and took the sorting path: 327 us, and 98 so. 1024 rows of 50257 at top_k 1000,
+// which fitted: 176.5 -> 173.)
+//
 // A row the list cannot hold (about 1.2 K values per 32768 of the row are
 // listed), whose threshold is not bounded this way (fewer than K finite
 // group maxima in its first two pieces, or a tie run over 64 keys), or whose
@@ -61,6 +69,7 @@ constexpr uint32_t kSPend = 512;             // listed values waiting for their 
 
 // misc[] slots
 enum : uint32_t { kSCandN = 0, kSDistinct = 1, kSFull = 2, kSPendN = 3, kSTau = 4, kSMisc = 5 };
+constexpr uint32_t kSRefShift = 14;  // key bits below a refined threshold's bin (1/512 of a value)
 
 struct StreamLds {
   __attribute__((aligned(16))) uint32_t coarse[kCoarseBins];
@@ -194,7 +203,7 @@ __device__ __forceinline__ void stream_rows(const SampleArgs& a, StreamKernelLds
     // (a row of another launch, or a finished generation).
     uint32_t outcome = 0u;
     // A row of another launch (a mixed call without the class table).
-    if (!a.row_cls_on && !(route_class(P, V) & a.row_class_mask)) outcome = 3u;
+    if (a.params && !a.row_cls_on && !(route_class(P, V) & a.row_class_mask)) outcome = 3u;
 
     const uint32_t len_b = ri.h0;
     const HistRow hr = FULL ? hist_row(a, b, ri.h0, ri.h1)
@@ -216,6 +225,9 @@ __device__ __forceinline__ void stream_rows(const SampleArgs& a, StreamKernelLds
       counts_moved = true;
     }
     const bool use_pen = rp != 1.0f && hr.H > 0u;
+    // Rows of a large K raise the threshold as they stream (below).
+    const bool refine = BIGK && stream_refines(K, V);
+    uint32_t* listed = reinterpret_cast<uint32_t*>(L.tmp);  // their histogram (the sort's buffer, free until then)
 
     if (outcome == 0u) {
       // 1. History multiplicities (order-independent integer LDS atomics)
@@ -230,6 +242,10 @@ __device__ __forceinline__ void stream_rows(const SampleArgs& a, StreamKernelLds
         for (uint32_t s = tid; s < kSBits; s += kBlock) L.hbits[s] = 0u;
       }
       lds_barrier();
+      // (Past the barrier, which wave 0 reaches only after the previous row's
+      // tail: that reads L.list and L.tmp.)
+      if (refine)
+        for (uint32_t i = tid; i < kFineBins; i += kBlock) listed[i] = 0u;
       if (use_pen) {
         for (uint32_t q = tid; q < hr.H; q += kBlock) {
           const uint32_t id = hr.at(q);
@@ -294,6 +310,7 @@ __device__ __forceinline__ void stream_rows(const SampleArgs& a, StreamKernelLds
       }
     };
     float tf = 0.0f;
+    uint32_t tkey = 0u;  // tf's key when the histogram of listed values starts
     // 4. Values at or above tf listed: unmarked ones by a wave scan of the
     //    per-thread counts, marked ones (rare) after their penalty, each
     //    taking a slot of its own.
@@ -327,6 +344,7 @@ __device__ __forceinline__ void stream_rows(const SampleArgs& a, StreamKernelLds
         const uint32_t i = 4u * (p * kSPieceQ + (e >> 2) * kBlock + tid) + (e & 3u);
         if (o < kSCand) L.list[o] = ((uint64_t)__float_as_uint(v) << 32) | i;
         ++o;
+        if (refine) atomicAdd(&listed[min((f2key(v) - tkey) >> kSRefShift, kFineBins - 1u)], 1u);
       }
       // Marked values wait in their own list: their penalty is applied once
       // the row is streamed (a penalty loop here would weigh on every
@@ -370,6 +388,7 @@ __device__ __forceinline__ void stream_rows(const SampleArgs& a, StreamKernelLds
         outcome = 1u;
       } else {
         tf = key2f(tlo);
+        tkey = tlo;
         // Pieces p (in A) and p + 1 (in Bf); each buffer reloads as soon as
         // it is listed, with the piece two ahead or, past this row's last,
         // with the next row's first two pieces (they land during this row's
@@ -393,6 +412,22 @@ __device__ __forceinline__ void stream_rows(const SampleArgs& a, StreamKernelLds
           } else if (jn < nrows) {
             stream_load(Bf, a.logits + (size_t)bn * a.ld, VL, 1u);
           }
+          if (refine) {
+            // The K-th largest of the unmarked values so far, to 1/512: every
+            // value of the row's top K lies at or above it too.
+            lds_barrier();
+            coarse_from_fine(listed, L.coarse);
+            lds_barrier();
+            if (wave == 0u) {
+              __builtin_amdgcn_s_setprio(3);
+              const uint32_t bin = hist_locate(L.coarse, listed, K, lane).lo >> 20;
+              const uint32_t t = bin ? lower_past_ties(tkey + (bin << kSRefShift), T, lane) : 0u;
+              if (lane == 0) L.misc[kSTau] = t;
+              __builtin_amdgcn_s_setprio(0);
+            }
+            lds_barrier();
+            tf = fmaxf(tf, key2f(max(L.misc[kSTau], tkey)));
+          }
         }
         fetched = true;
         // The row's last V - VL values, one thread each.
@@ -412,6 +447,32 @@ __device__ __forceinline__ void stream_rows(const SampleArgs& a, StreamKernelLds
         }
         LLMHIP_MARK(5);
         lds_barrier();
+        if (refine && L.misc[kSCandN] <= kSCand) {
+          // Only the listed values at or above the last threshold are sorted.
+          static_assert(kSCand == 4u * kBlock, "four per thread");
+          const uint32_t n0 = L.misc[kSCandN];
+          uint64_t r[4];
+          bool in[4];
+#pragma unroll
+          for (uint32_t q = 0; q < 4u; ++q) {
+            const uint32_t i = tid + q * kBlock;
+            r[q] = i < n0 ? L.list[i] : 0ull;
+            in[q] = i < n0 && __uint_as_float((uint32_t)(r[q] >> 32)) >= tf;
+          }
+          lds_barrier();
+          if (tid == 0) L.misc[kSCandN] = 0u;
+          lds_barrier();
+#pragma unroll
+          for (uint32_t q = 0; q < 4u; ++q) {
+            const uint64_t m = __ballot(in[q]);
+            if (m == 0ull) continue;
+            uint32_t o = 0u;
+            if (lane == 0) o = atomicAdd(&L.misc[kSCandN], (uint32_t)__popcll((unsigned long long)m));
+            o = readlane_u32(o, 0) + lanes_below(m);
+            if (in[q]) L.list[o] = r[q];
+          }
+          lds_barrier();
+        }
         // The marked values' penalties (generate.rs:343-352), stopping once
         // a value is below the threshold (exact for rp >= 1).
         const uint32_t npend = L.misc[kSPendN];

@@ -17,7 +17,7 @@ __global__ __launch_bounds__(kBlock) void sample_vocab_kernel(SampleArgs a) {
   } L;
   const uint32_t b = launch_row(a);
   if (b >= a.B) return;
-  if (!a.row_cls_on && !(route_class(load_params(a, b), a.V) & a.row_class_mask)) return;
+  if (a.params && !a.row_cls_on && !(route_class(load_params(a, b), a.V) & a.row_class_mask)) return;
   if (!vocab_row<PLAIN>(a, b, L.v, a.V >= 4u)) {
     if (threadIdx.x == 0) atomicAdd(a.handovers, 1u);
     __syncthreads();

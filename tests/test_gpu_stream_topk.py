@@ -174,3 +174,40 @@ def test_full_batches_at_small_k(sampler, cfg, k):
     g = _device_run(sampler, w, prm, want_probs=False)
     _check(g, w, prm, f"config{cfg} full k={k}", want_probs=False)
     assert g["handovers"] == 0
+
+
+# Rows whose K is above 256, or whose list would not hold 1.2 K values per
+# 32768, raise the threshold as they stream: both sides of K = 256 and of the
+# largest K taken (1169 at four parts, 940 at eight), the smallest vocabulary
+# and ragged ones. shape: normal, heavy-tailed, ascending (every part's values
+# above the last one's: the threshold rises with each), or few distinct values.
+@pytest.mark.parametrize("V,K,shape,handed", [
+    (32769, 257, "normal", 0), (32769, 1567, "normal", 0), (50257, 1000, "normal", 0), (65537, 900, "gumbel", 0),
+    (98304, 1169, "gumbel", 0), (131072, 256, "normal", 0), (131072, 257, "gumbel", 0), (131072, 820, "normal", 0),
+    (131072, 1169, "normal", 0), (131072, 1170, "normal", 0), (131071, 1000, "gumbel", 0), (262147, 940, "normal", 0),
+    (400001, 60, "normal", 0), (131072, 300, "ascending", None), (131072, 700, "coarse", None)])
+@pytest.mark.parametrize("extra", ["plain", "history", "mask"])
+def test_threshold_raised_while_streaming(sampler, V, K, shape, handed, extra):
+    rs = np.random.default_rng(V + K)
+    B = 4
+    x = rs.standard_normal((B, V)) if shape != "gumbel" else rs.gumbel(size=(B, V))
+    if shape == "ascending":
+        x = x + 6.0 * np.arange(V) / V
+    if shape == "coarse":
+        x = np.round(x * 4.0) / 4.0
+    w = make_workload(5, B=B, V=64)
+    w.logits, w.V, w.ld, w.hist, w.hist_offsets = x.astype(np.float32), V, V, None, None
+    rp, allowed = 1.0, None
+    if extra == "history":  # the row's own top ids and ids at random
+        rp, H = 1.25, 600
+        top = np.argsort(-w.logits, axis=1)[:, :2 * K]
+        hist = np.stack([np.concatenate([rs.choice(t, H // 2), rs.integers(0, V, H // 2)]) for t in top])
+        w.hist = hist.astype(np.uint32).reshape(-1)
+        w.hist_offsets = (np.arange(B + 1) * H).astype(np.uint32)
+    if extra == "mask":
+        allowed = (rs.random(V) < 0.5).astype(np.uint8)
+    prm = make_params(0.9, K, 0.999, 0.0, rp)
+    g = _device_run(sampler, w, prm, allowed=allowed)
+    _check(g, w, prm, f"V={V} K={K} {shape} {extra}", allowed=allowed)
+    if handed is not None:
+        assert g["handovers"] == handed
