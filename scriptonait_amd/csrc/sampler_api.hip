@@ -29,6 +29,7 @@ hipError_t launch_general(const SampleArgs& a, hipStream_t s);
 hipError_t launch_vocab(const SampleArgs& a, bool plain, hipStream_t s);
 hipError_t launch_seen_bits(const uint32_t* tokens, uint64_t n, uint32_t V, uint32_t* bits, hipStream_t s);
 hipError_t launch_take_status(uint32_t* words, hipStream_t s);
+hipError_t launch_host_status(uint32_t* word, uint32_t* out, hipStream_t s);
 hipError_t launch_stream(const SampleArgs& a, bool bigk, hipStream_t s);
 hipError_t launch_read_floor(const float* logits, uint64_t ld, uint32_t B, uint32_t V, int read, float* out,
                              hipStream_t s);
@@ -97,6 +98,28 @@ struct DevBuf {
   }
 };
 
+// A pinned host buffer that only grows: the GPU reads and writes it in place.
+struct HostBuf {
+  void* ptr = nullptr;
+  size_t cap = 0;
+  int ensure(size_t bytes) {
+    if (bytes <= cap) return LLMHIP_OK;
+    release();
+    const hipError_t e = hipHostMalloc(&ptr, bytes, hipHostMallocDefault);
+    if (e != hipSuccess) {
+      ptr = nullptr;
+      return hip_fail(e, "hipHostMalloc");
+    }
+    cap = bytes;
+    return LLMHIP_OK;
+  }
+  void release() {
+    if (ptr) (void)hipHostFree(ptr);
+    ptr = nullptr;
+    cap = 0;
+  }
+};
+
 }  // namespace
 
 struct llmhip_ctx {
@@ -111,6 +134,9 @@ struct llmhip_ctx {
   uint32_t cus = 0;              // the device's compute units (persistent launches take one workgroup each)
   // staging of the host entry
   DevBuf logits, hist, hoff, allowed, rng, ids, probs, kept;
+  HostBuf stage;    // a small host call's inputs and results
+  DevBuf stage_in;  // its inputs, for kernels that read a row more than once
+  bool host_word_set = false;  // a host call ended early: its flags may still be set
 };
 
 namespace {
@@ -374,6 +400,100 @@ int decode_step(llmhip_ctx* ctx, const float* logits, size_t B, size_t V, size_t
 
 }  // namespace
 
+namespace {
+
+// A host call's status, from the flags its kernels set.
+int host_flags(uint32_t flags) {
+  if (flags == 0) return LLMHIP_OK;
+  // A kernel hit an internal limit: its results are not trustworthy.
+  g_last_error = "internal error: a workgroup sync wait timed out in the sampler kernel";
+  return LLMHIP_ERR_HIP;
+}
+
+// Whether the register path, which reads each row once and all of it at once,
+// takes a row with these parameters.
+bool reads_row_once(const llmhip_params& p, size_t V) {
+  return V >= 4 && V <= kMaxFastV && (row_class(p, (uint32_t)V) & (kClassGreedy | kClassTopK)) != 0u;
+}
+
+// llmhip_sample_host for small inputs (kHostStageBytes in all) without
+// probabilities. Separate copies cost a host call each, and copies of a
+// caller's pageable memory wait for one another. Here the inputs are gathered
+// in pinned memory, which the register path's kernels read in place; the other
+// kernels, which read a row more than once or through one workgroup's few
+// loads in flight, get one copy of it. Results and RNG states are in pinned
+// memory too, and a last small kernel puts the call's flags there and clears
+// them for the next call.
+// One row of 32000 with a mask and a history: 144-152 us with separate copies,
+// 36 so; 16 rows: 208 and 98; 64: 387 and 295; 128: 600 and 650, which sets
+// the limit.
+constexpr size_t kHostStageBytes = 8u << 20;
+
+int sample_host_small(llmhip_ctx* ctx, const float* logits, size_t B, size_t V, size_t ld,
+                      const llmhip_params* params, size_t params_stride, const uint32_t* hist, size_t nhist,
+                      const uint32_t* hist_offsets, const uint8_t* allowed, size_t allowed_len, uint32_t eos_id,
+                      uint64_t* rng_state, uint32_t* out_ids, uint32_t* out_kept, size_t bytes, hipStream_t s,
+                      uint32_t* kstatus) {
+  // inputs: logits | history | offsets | mask | params; then, always pinned:
+  // RNG states | ids | kept | flags. Parts start 256 bytes apart or more (bytes
+  // leaves room for that).
+  int st = ctx->stage.ensure(bytes);
+  if (st) return st;
+  uint8_t* const base = static_cast<uint8_t*>(ctx->stage.ptr);
+  size_t at = 0;
+  auto part = [&](size_t n) {
+    const size_t o = at;
+    at += (n + 255u) / 256u * 256u;
+    return o;
+  };
+  const size_t nparams = params_stride ? (B - 1) * params_stride + 1 : 0;
+  const size_t o_log = part(B * V * sizeof(float)), o_hist = part(nhist * sizeof(uint32_t)),
+               o_off = part(hist ? (B + 1) * sizeof(uint32_t) : 0), o_mask = part(allowed_len),
+               o_prm = part(nparams * sizeof(llmhip_params)), in_bytes = at;
+  const size_t o_rng = part(B * sizeof(uint64_t)), o_ids = part(B * sizeof(uint32_t)),
+               o_kept = part(out_kept ? B * sizeof(uint32_t) : 0), o_status = part(sizeof(uint32_t));
+  if (at > ctx->stage.cap) return arg_fail("internal error: host staging size");
+  for (size_t b = 0; b < B; ++b) memcpy(base + o_log + b * V * sizeof(float), logits + b * ld, V * sizeof(float));
+  if (nhist) memcpy(base + o_hist, hist, nhist * sizeof(uint32_t));
+  if (hist) memcpy(base + o_off, hist_offsets, (B + 1) * sizeof(uint32_t));
+  if (allowed_len) memcpy(base + o_mask, allowed, allowed_len);
+  if (nparams) memcpy(base + o_prm, params, nparams * sizeof(llmhip_params));
+  memcpy(base + o_rng, rng_state, B * sizeof(uint64_t));
+
+  bool once = true;
+  for (size_t b = 0; b < (params_stride ? B : 1) && once; ++b) once = reads_row_once(params[b * params_stride], V);
+  const uint8_t* in = base;
+  if (!once) {
+    if ((st = ctx->stage_in.ensure(in_bytes))) return st;
+    HIP_TRY(hipMemcpyAsync(ctx->stage_in.ptr, base, in_bytes, hipMemcpyHostToDevice, s));
+    in = static_cast<const uint8_t*>(ctx->stage_in.ptr);
+  }
+  Mask m;
+  m.bytes = allowed_len ? in + o_mask : nullptr;
+  m.len = allowed_len;
+  st = enqueue(ctx, reinterpret_cast<const float*>(in + o_log), B, V, V, params, params_stride,
+               nparams ? reinterpret_cast<const llmhip_params*>(in + o_prm) : nullptr,
+               hist ? reinterpret_cast<const uint32_t*>(in + o_hist) : nullptr,
+               hist ? reinterpret_cast<const uint32_t*>(in + o_off) : nullptr, m, eos_id,
+               reinterpret_cast<uint64_t*>(base + o_rng), reinterpret_cast<uint32_t*>(base + o_ids), nullptr,
+               out_kept ? reinterpret_cast<uint32_t*>(base + o_kept) : nullptr, s, true);
+  if (st == LLMHIP_OK) {
+    const hipError_t e = launch_host_status(static_cast<uint32_t*>(ctx->status.ptr) + kStatusHostWord,
+                                            reinterpret_cast<uint32_t*>(base + o_status), s);
+    if (e != hipSuccess) st = hip_fail(e, "launch_host_status");
+  }
+  const hipError_t e = hipStreamSynchronize(s);
+  if (st) return st;
+  if (e != hipSuccess) return hip_fail(e, "hipStreamSynchronize");
+  memcpy(out_ids, base + o_ids, B * sizeof(uint32_t));
+  memcpy(rng_state, base + o_rng, B * sizeof(uint64_t));
+  if (out_kept) memcpy(out_kept, base + o_kept, B * sizeof(uint32_t));
+  memcpy(kstatus, base + o_status, sizeof(uint32_t));
+  return LLMHIP_OK;
+}
+
+}  // namespace
+
 extern "C" {
 
 int llmhip_abi_version(void) { return LLMHIP_ABI_VERSION; }
@@ -441,6 +561,8 @@ int llmhip_ctx_destroy(llmhip_ctx* ctx) {
   for (DevBuf* b : {&ctx->scratch, &ctx->params, &ctx->status, &ctx->head_logits,
                     &ctx->logits, &ctx->hist, &ctx->hoff, &ctx->allowed, &ctx->rng, &ctx->ids, &ctx->probs, &ctx->kept})
     b->release();
+  ctx->stage_in.release();
+  ctx->stage.release();
   if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
   delete ctx;
   return LLMHIP_OK;
@@ -621,15 +743,31 @@ int llmhip_sample_host(llmhip_ctx* ctx, const float* logits, size_t B, size_t V,
   if (!d.ok) return hip_fail(hipErrorInvalidDevice, "hipSetDevice");
   hipStream_t s = ctx->stream;
   uint32_t* host_word = static_cast<uint32_t*>(ctx->status.ptr) + kStatusHostWord;
-  // This call reports only what its own kernels flag.
-  HIP_TRY(hipMemsetAsync(host_word, 0, sizeof(uint32_t), s));
-
-  // Rows are copied densely (ld = V on the device).
+  // The word is clear between calls (each takes what its own kernels flagged),
+  // unless one ended early.
+  if (ctx->host_word_set) HIP_TRY(hipMemsetAsync(host_word, 0, sizeof(uint32_t), s));
   const size_t nlog = B * V;
   const size_t nhist = hist ? (size_t)hist_offsets[B] : 0;
   if (hist && hist_offsets[0] != 0) return arg_fail("hist_offsets[0] must be 0");
   for (size_t b = 0; hist && b < B; ++b)
     if (hist_offsets[b + 1] < hist_offsets[b]) return arg_fail("hist_offsets must be non-decreasing");
+  uint32_t kstatus = 0;
+  if (V > 0 && !out_probs && B <= kHostStageBytes / 64u && params_stride <= kHostStageBytes / 64u &&
+      V <= kHostStageBytes / sizeof(float)) {
+    const size_t bytes = nlog * sizeof(float) + (nhist + 1) * sizeof(uint32_t) + allowed_len +
+                         B * (params_stride * sizeof(llmhip_params) + 24u) + 9u * 256u;
+    if (bytes <= kHostStageBytes) {
+      ctx->host_word_set = true;
+      st = sample_host_small(ctx, logits, B, V, ld, params, params_stride, hist, nhist, hist_offsets, allowed,
+                             allowed_len, eos_id, rng_state, out_ids, out_kept, bytes, s, &kstatus);
+      if (st) return st;
+      ctx->host_word_set = false;
+      return host_flags(kstatus);
+    }
+  }
+  ctx->host_word_set = true;
+
+  // Rows are copied densely (ld = V on the device).
   if ((st = ctx->logits.ensure(nlog * sizeof(float)))) return st;
   if ((st = ctx->rng.ensure(B * sizeof(uint64_t)))) return st;
   if ((st = ctx->ids.ensure(B * sizeof(uint32_t)))) return st;
@@ -676,15 +814,11 @@ int llmhip_sample_host(llmhip_ctx* ctx, const float* logits, size_t B, size_t V,
   HIP_TRY(hipMemcpyAsync(rng_state, ctx->rng.ptr, B * sizeof(uint64_t), hipMemcpyDeviceToHost, s));
   if (out_kept) HIP_TRY(hipMemcpyAsync(out_kept, ctx->kept.ptr, B * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
   if (out_probs) HIP_TRY(hipMemcpyAsync(out_probs, ctx->probs.ptr, nlog * sizeof(float), hipMemcpyDeviceToHost, s));
-  uint32_t kstatus = 0;
   HIP_TRY(hipMemcpyAsync(&kstatus, host_word, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+  HIP_TRY(hipMemsetAsync(host_word, 0, sizeof(uint32_t), s));
   HIP_TRY(hipStreamSynchronize(s));
-  if (kstatus) {
-    // A kernel hit an internal limit: its results are not trustworthy.
-    g_last_error = "internal error: a workgroup sync wait timed out in the sampler kernel";
-    return LLMHIP_ERR_HIP;
-  }
-  return LLMHIP_OK;
+  ctx->host_word_set = false;
+  return host_flags(kstatus);
 }
 
 int llmhip_decode_step(llmhip_ctx* ctx, const float* logits, size_t B, size_t V, size_t ld,

@@ -113,6 +113,16 @@ __global__ void take_status_kernel(uint32_t* words) {
   }
 }
 
+// A host call's flags, moved to its pinned result and cleared.
+__global__ void host_status_kernel(uint32_t* word, uint32_t* out) {
+  if (threadIdx.x == 0 && blockIdx.x == 0) *out = atomicExch(word, 0u);
+}
+
+hipError_t launch_host_status(uint32_t* word, uint32_t* out, hipStream_t s) {
+  hipLaunchKernelGGL(host_status_kernel, dim3(1), dim3(64), 0, s, word, out);
+  return hipGetLastError();
+}
+
 hipError_t launch_take_status(uint32_t* words, hipStream_t s) {
   hipLaunchKernelGGL(take_status_kernel, dim3(1), dim3(64), 0, s, words);
   return hipGetLastError();

@@ -109,3 +109,34 @@ def test_generation_loop_with_windowed_history():
                                  cfg.repetition_penalty, recent, ref)
         assert got == want
         tokens.append(got)
+
+
+@pytest.mark.parametrize("B,V,ld", [(1, 1, 1), (1, 3, 3), (1, 32000, 32000), (3, 32769, 32771), (64, 32000, 32000),
+                                    (65, 32000, 32004), (5, 4099, 5000)])
+@pytest.mark.parametrize("top_k,per_row", [(40, False), (0, False), (2000, True)])
+def test_host_calls_on_both_sides_of_the_staging_limit(sampler, B, V, ld, top_k, per_row):
+    """The host entry gathers small calls in pinned memory and copies larger
+    ones part by part (64 rows of 32000 lie on one side, 65 on the other):
+    dense and strided rows, every kernel, shared and per-row parameters; a
+    second call on other inputs sees only its own."""
+    from oracle import oracle
+    from scriptonait_amd.workloads import PARAMS_DTYPE
+
+    rs = np.random.default_rng(B * V + top_k)
+    for call in range(2):
+        x = rs.standard_normal((B, ld)).astype(np.float32) * 2
+        H = int(rs.integers(0, 200))
+        hist = rs.integers(0, V + 2, B * H).astype(np.uint32)
+        offs = (np.arange(B + 1) * H).astype(np.uint32)
+        allowed = (rs.random(V + 1 - call) < 0.8).astype(np.uint8)
+        prm = np.zeros(B if per_row else 1, dtype=PARAMS_DTYPE)
+        prm["temperature"], prm["top_k"], prm["top_p"], prm["repetition_penalty"] = 0.8, top_k, 0.95, 1.1
+        if per_row:
+            prm["temperature"][::3] = 0.0
+            prm["top_k"][1::3] = 30
+        seeds = rs.integers(0, 2**63, size=B, dtype=np.uint64)
+        g = sampler.sample_host(x, prm, seeds, hist, offs, allowed=allowed, V=V)
+        o = oracle.sample_batch(x, prm, seeds, hist, offs, allowed=allowed, V=V, threads=8)
+        assert np.array_equal(g.ids, o.ids)
+        assert np.array_equal(g.kept, o.kept)
+        assert np.array_equal(g.rng_state, o.rng_state)
