@@ -73,6 +73,10 @@ constexpr uint32_t kCoarseBins = 256;             // key bits 31..24
 constexpr uint32_t kFineBins = 4096;              // key bits 31..20
 constexpr uint32_t kTauWaves = 8;                 // waves whose maxima form the threshold sample
 constexpr uint32_t kSpecNum = 8, kSpecDen = 5;    // the threshold aims at ~(kSpecNum/kSpecDen)*K values
+// Fewer than K / kUndercut survivors: the second speculative pass, four times
+// as deep at most, would find too few as well (4 us for a row of a saturated
+// window), and the proven threshold follows at once.
+constexpr uint32_t kUndercut = 32;
 constexpr uint32_t kSpecMaxK = 384;               // larger K: the scan entries would overflow; proven threshold
 constexpr uint32_t kRefineCount = 16;             // a fine bin holding more keys is split once more
 constexpr uint32_t kSortedK = 1024;               // K up to which the sorted top K is copied to skey/sid
@@ -92,6 +96,9 @@ constexpr int kCandN2 = 10;    // candidates of the second speculative pass
 constexpr int kOverflow2 = 11; // some wave's region overflowed in it
 constexpr int kTau2 = 12;      // its threshold key (1: no second pass)
 constexpr int kTau0 = 13;      // the proven threshold key (1: not bounded here)
+constexpr uint32_t kSplitBin = 2u;  // in kTau0: its fine bin (below) is split once more
+constexpr int kCrowdBin = 14;  // that bin's lower edge
+constexpr int kCrowdNeed = 15; // the rank inside that bin
 
 // BIGK: the large-K kernel's scan entries hold 128 per wave (a proven
 // threshold for K up to 1024 puts about 1.2 K chunks in them).
@@ -1119,7 +1126,7 @@ __device__ __forceinline__ bool fast_row(const SampleArgs& a, FastLds<NCH, BIGK>
   // deep enough for the 5K/4 - n survivors still missing (at most 8 times
   // the first). One wave selects it (a selection in every wave would compete
   // for the ALUs).
-  if (__builtin_expect(spec && n < K && !ovf, 0)) {
+  if (__builtin_expect(spec && n < K && n >= K / kUndercut && !ovf, 0)) {
     if (wave == 0u) {
       __builtin_amdgcn_s_setprio(3);  // as for the first threshold
       const uint64_t q = spec_q(L.misc[kSampled]);
@@ -1183,6 +1190,7 @@ __device__ __forceinline__ bool fast_row(const SampleArgs& a, FastLds<NCH, BIGK>
     }
     slot_n = kCandN;
     slot_o = kOverflow;
+    float kmx = -INFINITY;  // this thread's known maximum
     if (by_chunk) {
 #pragma unroll
       for (int c = 0; c < NCH; ++c) {
@@ -1193,8 +1201,8 @@ __device__ __forceinline__ bool fast_row(const SampleArgs& a, FastLds<NCH, BIGK>
         if (cm > -INFINITY) atomicAdd(&L.fine[f2key(cm) >> 20], 1u);
       }
     } else {
-      const float tm = known_max(pmr);
-      if (tm > -INFINITY) atomicAdd(&L.fine[f2key(tm) >> 20], 1u);
+      kmx = known_max(pmr);
+      if (kmx > -INFINITY) atomicAdd(&L.fine[f2key(kmx) >> 20], 1u);
     }
     lds_barrier();
     coarse_from_fine(L.fine, L.coarse);
@@ -1203,24 +1211,66 @@ __device__ __forceinline__ bool fast_row(const SampleArgs& a, FastLds<NCH, BIGK>
     // (hist_locate's 0 says fewer than K threads hold a known value).
     if (wave == 0u) {
       __builtin_amdgcn_s_setprio(3);  // as for the first threshold
-      const uint32_t t0 = hist_locate(L.coarse, L.fine, K, lane).lo;
+      const HistPos h0 = hist_locate(L.coarse, L.fine, K, lane);
+      const uint32_t t0 = h0.lo;
+      // A crowded bin (1/8 of a value wide: the K-th largest known value of a
+      // row whose top ids are all in the history lies in a dense part of the
+      // row) is split once more, below; 256 rows of 32000 at K = 64 whose
+      // windows are full of their own draws: 37.8 us without, 20.8 with (24 of
+      // the rows then listed over 512 values and took the per-slot narrowing
+      // below). At over 4 K values in place of 2 K: 28-30 us.
+      const bool crowded = !by_chunk && t0 != 0u && K - h0.need + h0.cnt > 2u * K + kRefineCount;
       // A large K goes to the per-slot narrowing below, which needs only
       // some key at or below its K-th largest known value: t0, or, when
       // fewer than K chunks hold a known value, the lowest finite key.
-      const uint32_t tk = huge ? (t0 ? t0 : 0x00800000u) : t0 ? lower_past_ties(t0, T, lane) : 0u;
+      uint32_t tk;
+      if (crowded) {
+        tk = kSplitBin;
+        if (lane == 0u) {
+          L.misc[kCrowdBin] = t0;
+          L.misc[kCrowdNeed] = h0.need;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+      } else {
+        tk = huge ? (t0 ? t0 : 0x00800000u) : t0 ? lower_past_ties(t0, T, lane) : 0u;
+      }
       (void)lds_publish(&L.misc[kTau0], tk ? tk : 1u);
       __builtin_amdgcn_s_setprio(0);
     }
-    const uint32_t tk0 = lds_wait_nonzero(&L.misc[kTau0], 1u, a);
+    uint32_t tk0 = lds_wait_nonzero(&L.misc[kTau0], 1u, a);
     if (tk0 <= 1u) return false;
+    if (tk0 == kSplitBin) {
+      const uint32_t crowd = L.misc[kCrowdBin];
+      reinterpret_cast<uint4*>(L.fine)[tid] = make_uint4(0u, 0u, 0u, 0u);
+      lds_barrier();
+      const uint32_t k = f2key(kmx);
+      if (kmx > -INFINITY && (k >> 20) == (crowd >> 20)) atomicAdd(&L.fine[(k << 12) >> 20], 1u);
+      lds_barrier();
+      coarse_from_fine(L.fine, L.coarse);
+      lds_barrier();
+      // Every wave selects (no second wait); the bin holds kCrowdNeed of them.
+      tk0 = lower_past_ties(crowd | (hist_locate(L.coarse, L.fine, L.misc[kCrowdNeed], lane).lo >> 12), T, lane);
+      if (tk0 == 0u) return false;
+    }
     LLMHIP_MARK(12);
     tf = key2f(tk0);
     // A large K puts more values at or above t0 than the scan entries hold.
     if (!huge) {
-      nent = 0u;
+      // A window that holds many of the row's top ids can put more chunks at
+      // or above t0 than the wave's entries hold (most of their values then
+      // fall to the penalty): the wave takes as many as fit at a time.
+      uint32_t left = (1u << NCH) - 1u;  // chunks to scan (uniform)
+      do {
+        nent = 0u;
 #pragma unroll
-      for (int c = 0; c < NCH; ++c) scan_chunk(c, mc[c]);
-      settle();
+        for (int c = 0; c < NCH; ++c) {
+          if (((left >> c) & 1u) && nent + (uint32_t)__popcll((unsigned long long)__ballot(mc[c] >= tf)) <= kEnt) {
+            scan_chunk(c, mc[c]);
+            left &= ~(1u << c);
+          }
+        }
+        settle();
+      } while (left != 0u);
       lds_barrier();
       LLMHIP_MARK(13);
       n = L.misc[kCandN];
@@ -1342,14 +1392,17 @@ __device__ __forceinline__ bool fast_row(const SampleArgs& a, FastLds<NCH, BIGK>
       const uint64_t* srt = n <= 2u * kBlock   ? sort_desc_lds<2>(lst, L.big_tmp, n)
                             : n <= 4u * kBlock ? sort_desc_lds<4>(lst, L.big_tmp, n)
                                                : sort_desc_lds<8>(lst, L.big_tmp, n);
+      LLMHIP_MARK(10);
       float* buf = srt == L.big_tmp ? reinterpret_cast<float*>(big_list(L)) : reinterpret_cast<float*>(L.big_tmp);
       auto key_at = [&](uint32_t i) { return (uint32_t)(srt[i] >> 32); };
       // The tail's terms are staged by every wave.
       stage_exp_terms(buf, K, key_at, L.exptab, tid, kBlock);
       lds_barrier();
+      LLMHIP_MARK(7);
       if (wave == 0)
         draw_tail_lds<true>(a, b, len_b, P, K, key_at, [&](uint32_t i) { return ~(uint32_t)srt[i]; }, rng0, L.exptab,
                             buf);
+      LLMHIP_MARK(8);
       return true;
     }
   }
