@@ -88,8 +88,9 @@ int llmhip_ctx_destroy(llmhip_ctx* ctx);
 /*
  * Batched sample_with on HOST buffers (replaces generate.rs:325-420 at its
  * call sites generate.rs:159 and crates/wasm-app/src/inference.rs:327).
- * Copies the inputs to the device, runs the kernels, copies the results
- * back and synchronizes before returning, so results are visible like the
+ * Brings the inputs to the device (small calls through pinned memory that
+ * the context keeps), runs the kernels, brings the results back and
+ * synchronizes before returning, so results are visible like the
  * reference's return value.
  *
  *   logits        [B][ld] f32, row b's V logits start at logits + b*ld (ld >= V)
