@@ -621,12 +621,22 @@ __device__ __forceinline__ bool fast_row(const SampleArgs& a, FastLds<NCH, BIGK>
   const bool has_hist = ring || (a.hist_offsets && a.hist);
   constexpr bool cmode = CMODE;  // multiplicities from the count table
   const uint32_t l7 = lane & 7u;
-  const uint32_t* hvsrc = ring ? (l7 == 1u && a.done ? a.done + b
-                                  : l7 == 2u && a.hist_start ? a.hist_start + b
-                                  : (l7 == 3u || l7 == 4u) && cmode ? a.counted + 2u * b + (l7 - 3u)
-                                  : a.ring_len + b)
-                               : (has_hist ? a.hist_offsets + b + (lane & 1u) : reinterpret_cast<const uint32_t*>(a.logits));
-  const uint32_t hv = *hvsrc;
+  // (A base and an index by selects: one conditional expression over whole
+  // pointers compiles to a tree of branches ahead of the row's loads.)
+  const uint32_t* hvsrc = reinterpret_cast<const uint32_t*>(a.logits);
+  uint32_t hvat = 0u;
+  if (ring) {
+    hvsrc = l7 == 1u && a.done ? a.done : l7 == 2u && a.hist_start ? a.hist_start : a.ring_len;
+    hvat = b;
+    if (cmode && (l7 == 3u || l7 == 4u)) {
+      hvsrc = a.counted;
+      hvat = 2u * b + (l7 - 3u);
+    }
+  } else if (has_hist) {
+    hvsrc = a.hist_offsets;
+    hvat = b + (lane & 1u);
+  }
+  const uint32_t hv = hvsrc[hvat];
   const uint32_t rv = reinterpret_cast<const uint32_t*>(a.rng_state + b)[lane & 1u];
   const uint32_t pw =
       a.params ? reinterpret_cast<const uint32_t*>(a.params + (size_t)b * a.params_stride)[min(lane, 4u)] : 0u;
@@ -885,9 +895,14 @@ __device__ __forceinline__ bool fast_row(const SampleArgs& a, FastLds<NCH, BIGK>
   // lower bound on its final maximum that needs no penalty.
   auto known_max = [&](uint32_t pmv) __attribute__((always_inline)) {
     float kv = -INFINITY;
+    // (A fresh copy, as in the per-slot narrowing below: where mkbits is the
+    // constant 0 the 32 per-slot bits would be shared with the loops there
+    // and live through the hot path, 44 spilled scalars at 8 chunks.)
+    uint32_t out = pmv | mkbits;
+    asm volatile("" : "+v"(out));
 #pragma unroll
     for (int e = 0; e < NCH * 4; ++e)
-      if ((((pmv | mkbits) >> e) & 1u) == 0u) kv = fmaxf(kv, x[e]);
+      if (((out >> e) & 1u) == 0u) kv = fmaxf(kv, x[e]);
     return kv;
   };
 
