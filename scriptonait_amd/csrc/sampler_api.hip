@@ -10,6 +10,7 @@
 #include <mutex>
 #include <string>
 
+#include "grow_buf.h"
 #include "sampler_common.h"
 
 // Device memory of llmhip_sample_device_noalloc, for callers that cannot
@@ -70,55 +71,31 @@ int arg_fail(const char* what) {
     if (e_ != hipSuccess) return hip_fail(e_, #expr); \
   } while (0)
 
-// A device buffer that only grows.
-struct DevBuf {
-  void* ptr = nullptr;
-  size_t cap = 0;
-  int ensure(size_t bytes) {
-    if (bytes <= cap) return LLMHIP_OK;
-    if (ptr) {
-      hipError_t e = hipFree(ptr);
-      ptr = nullptr;
-      cap = 0;
-      if (e != hipSuccess) return hip_fail(e, "hipFree");
-    }
-    size_t want = std::max<size_t>(bytes, 256);
-    hipError_t e = hipMalloc(&ptr, want);
-    if (e != hipSuccess) {
-      ptr = nullptr;
-      return hip_fail(e, "hipMalloc");
-    }
-    cap = want;
-    return LLMHIP_OK;
+struct DeviceMem {
+  static int alloc(void** p, size_t bytes) {
+    const hipError_t e = hipMalloc(p, bytes);
+    return e == hipSuccess ? LLMHIP_OK : hip_fail(e, "hipMalloc");
   }
-  void release() {
-    if (ptr) (void)hipFree(ptr);
-    ptr = nullptr;
-    cap = 0;
+  static int free(void* p) {
+    const hipError_t e = hipFree(p);
+    return e == hipSuccess ? LLMHIP_OK : hip_fail(e, "hipFree");
   }
 };
 
-// A pinned host buffer that only grows: the GPU reads and writes it in place.
-struct HostBuf {
-  void* ptr = nullptr;
-  size_t cap = 0;
-  int ensure(size_t bytes) {
-    if (bytes <= cap) return LLMHIP_OK;
-    release();
-    const hipError_t e = hipHostMalloc(&ptr, bytes, hipHostMallocDefault);
-    if (e != hipSuccess) {
-      ptr = nullptr;
-      return hip_fail(e, "hipHostMalloc");
-    }
-    cap = bytes;
-    return LLMHIP_OK;
+// Pinned host memory: the GPU reads and writes it in place.
+struct PinnedMem {
+  static int alloc(void** p, size_t bytes) {
+    const hipError_t e = hipHostMalloc(p, bytes, hipHostMallocDefault);
+    return e == hipSuccess ? LLMHIP_OK : hip_fail(e, "hipHostMalloc");
   }
-  void release() {
-    if (ptr) (void)hipHostFree(ptr);
-    ptr = nullptr;
-    cap = 0;
+  static int free(void* p) {
+    const hipError_t e = hipHostFree(p);
+    return e == hipSuccess ? LLMHIP_OK : hip_fail(e, "hipHostFree");
   }
 };
+
+using DevBuf = GrowBuf<DeviceMem>;
+using HostBuf = GrowBuf<PinnedMem>;
 
 }  // namespace
 
@@ -427,7 +404,7 @@ bool reads_row_once(const llmhip_params& p, size_t V) {
 // One row of 32000 with a mask and a history: 144-152 us with separate copies,
 // 36 so; 16 rows: 208 and 98; 64: 387 and 295; 128: 600 and 650, which sets
 // the limit.
-constexpr size_t kHostStageBytes = 8u << 20;
+constexpr size_t kHostStageBytes = kRoundedBytes;
 
 int sample_host_small(llmhip_ctx* ctx, const float* logits, size_t B, size_t V, size_t ld,
                       const llmhip_params* params, size_t params_stride, const uint32_t* hist, size_t nhist,
