@@ -707,7 +707,7 @@ __device__ __forceinline__ bool fast_row(const SampleArgs& a, FastLds<NCH, BIGK>
   const float T = P.temperature, rp = P.repetition_penalty;
   const HistRow hr = hist_row(a, b, h0, h1);
   const uint32_t H = rp != 1.0f ? hr.H : 0u;
-  const bool use_pen = H > 0 && H < 65536u;
+  const bool use_pen = H > 0 && H < kCountedHistory;
   // This wave's share of the count table (only when a history may be used).
   if (a.hist) {
     uint4* c4 = reinterpret_cast<uint4*>(L.cnt);
@@ -797,7 +797,7 @@ __device__ __forceinline__ bool fast_row(const SampleArgs& a, FastLds<NCH, BIGK>
   auto slide_before_handover = [&]() __attribute__((always_inline)) {
     if (cmode && !cplan.rebuild && wave == 0) counts_slide(a, b, cplan);
   };
-  if (__builtin_expect(H >= 65536u, 0)) {  // a u16 multiplicity could overflow
+  if (__builtin_expect(H >= kCountedHistory, 0)) {
     slide_before_handover();
     return false;
   }

@@ -388,9 +388,16 @@ int host_flags(uint32_t flags) {
 }
 
 // Whether the register path, which reads each row once and all of it at once,
-// takes a row with these parameters.
-bool reads_row_once(const llmhip_params& p, size_t V) {
-  return V >= 4 && V <= kMaxFastV && (row_class(p, (uint32_t)V) & (kClassGreedy | kClassTopK)) != 0u;
+// takes a row with these parameters and H history ids. Rows that it hands to
+// the sorting path (a penalty below 1) read their history several times, so a
+// long one is copied (32000 logits, 60000 ids: 304 us in place, 176 copied; 4096
+// ids: 66 us in place).
+bool reads_row_once(const llmhip_params& p, size_t V, uint32_t H) {
+  const uint32_t cls = row_class(p, (uint32_t)V);
+  if (V < 4 || V > kMaxFastV || !(cls & (kClassGreedy | kClassTopK))) return false;
+  if (p.repetition_penalty == 1.0f) return true;  // the history is not read
+  const bool kept = cls == kClassGreedy || p.repetition_penalty >= 1.0f;
+  return H < (kept ? kCountedHistory : 8192u);
 }
 
 // llmhip_sample_host for small inputs (kHostStageBytes in all) without
@@ -403,7 +410,8 @@ bool reads_row_once(const llmhip_params& p, size_t V) {
 // them for the next call.
 // One row of 32000 with a mask and a history: 144-152 us with separate copies,
 // 36 so; 16 rows: 208 and 98; 64: 387 and 295; 128: 600 and 650, which sets
-// the limit.
+// the limit. A history that the register path cannot count, 65536 ids: 279 us
+// with separate copies, 189 with one, 335 read in place; 131072: 404, 314, 610.
 constexpr size_t kHostStageBytes = kRoundedBytes;
 
 int sample_host_small(llmhip_ctx* ctx, const float* logits, size_t B, size_t V, size_t ld,
@@ -438,7 +446,8 @@ int sample_host_small(llmhip_ctx* ctx, const float* logits, size_t B, size_t V, 
   memcpy(base + o_rng, rng_state, B * sizeof(uint64_t));
 
   bool once = true;
-  for (size_t b = 0; b < (params_stride ? B : 1) && once; ++b) once = reads_row_once(params[b * params_stride], V);
+  for (size_t b = 0; b < B && once; ++b)
+    once = reads_row_once(params[b * params_stride], V, hist ? hist_offsets[b + 1] - hist_offsets[b] : 0u);
   const uint8_t* in = base;
   if (!once) {
     if ((st = ctx->stage_in.ensure(in_bytes))) return st;

@@ -396,6 +396,10 @@ __host__ __device__ __forceinline__ bool stream_takes(const llmhip_params& p, ui
   return (uint64_t)p.top_k * (147u + 50u * (m - 1u)) <= (uint64_t)kStreamCand * 15u / 16u * 60u;
 }
 
+// A longer history goes from the register path to the sorting path: a u16
+// multiplicity could overflow.
+constexpr uint32_t kCountedHistory = 65536;
+
 // The path a row is routed to: its class, except that a top-k row past the
 // register path that the streaming path does not take goes with the
 // kClassFull rows (the sorting path, which selects any K <= kSelCap).
