@@ -73,10 +73,11 @@ constexpr uint32_t kCoarseBins = 256;             // key bits 31..24
 constexpr uint32_t kFineBins = 4096;              // key bits 31..20
 constexpr uint32_t kTauWaves = 8;                 // waves whose maxima form the threshold sample
 constexpr uint32_t kSpecNum = 8, kSpecDen = 5;    // the threshold aims at ~(kSpecNum/kSpecDen)*K values
-// Fewer than K / kUndercut survivors: the second speculative pass, four times
-// as deep at most, would find too few as well (4 us for a row of a saturated
-// window), and the proven threshold follows at once.
-constexpr uint32_t kUndercut = 32;
+// Fewer than K / 32 survivors: the second speculative pass, four times as deep
+// at most, would find too few as well (4 us for a row of a saturated window),
+// and the proven threshold follows at once.
+constexpr bool second_pass_pays(uint32_t n, uint32_t K) { return n * 32u >= K; }
+static_assert(!second_pass_pays(0u, 1u) && second_pass_pays(1u, 32u) && !second_pass_pays(1u, 33u), "at every K");
 constexpr uint32_t kSpecMaxK = 384;               // larger K: the scan entries would overflow; proven threshold
 constexpr uint32_t kRefineCount = 16;             // a fine bin holding more keys is split once more
 constexpr uint32_t kSortedK = 1024;               // K up to which the sorted top K is copied to skey/sid
@@ -1141,7 +1142,7 @@ __device__ __forceinline__ bool fast_row(const SampleArgs& a, FastLds<NCH, BIGK>
   // deep enough for the 5K/4 - n survivors still missing (at most 8 times
   // the first). One wave selects it (a selection in every wave would compete
   // for the ALUs).
-  if (__builtin_expect(spec && n < K && n >= K / kUndercut && !ovf, 0)) {
+  if (__builtin_expect(spec && n < K && second_pass_pays(n, K) && !ovf, 0)) {
     if (wave == 0u) {
       __builtin_amdgcn_s_setprio(3);  // as for the first threshold
       const uint64_t q = spec_q(L.misc[kSampled]);
