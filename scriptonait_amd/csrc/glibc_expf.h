@@ -73,16 +73,42 @@ LLMHIP_HD uint64_t f64_bits(double x) {
   return u;
 }
 
-// exp of a binary32 value, bit-identical to glibc 2.35's expf (FMA variant),
-// with the 2^(i/32) table read from `tab` (kExp2fTab, or a copy of it that a
-// kernel staged in LDS so the lookup never waits behind streaming loads).
-LLMHIP_HD float glibc_expf_tab(float x, const uint64_t* tab) {
+// The steps of glibc 2.35's expf (FMA variant) for |x| < 88, with the 2^(i/32)
+// table read from `tab` (kExp2fTab, or a copy of it that a kernel staged in LDS
+// so the lookup never waits behind streaming loads): callers that know their
+// range take it without the tests for its ends.
+LLMHIP_HD float glibc_expf_mid(float x, const uint64_t* tab) {
   const double kInvLn2N = 0x1.71547652b82fep+0 * 32.0;
   const double kShift = 0x1.8p+52;
   const double kC0 = 0x1.c6af84b912394p-5 / (32.0 * 32.0 * 32.0);
   const double kC1 = 0x1.ebfce50fac4f3p-3 / (32.0 * 32.0);
   const double kC2 = 0x1.62e42ff0c52d6p-1 / 32.0;
 
+  const double xd = (double)x;
+#if LLMHIP_EXPF_FUSED
+  double kd = __builtin_fma(kInvLn2N, xd, kShift);
+#else
+  double z = kInvLn2N * xd;
+  double kd = z + kShift;
+#endif
+  const uint32_t ki = (uint32_t)f64_bits(kd);
+  kd -= kShift;
+  const uint64_t t = tab[ki % 32u];  // + ki << 47, which reaches the upper word only
+  const double s = f64_from_bits(((uint64_t)((uint32_t)(t >> 32) + (ki << 15)) << 32) | (uint32_t)t);
+#if LLMHIP_EXPF_FUSED
+  const double r = __builtin_fma(kInvLn2N, xd, -kd);
+  const double z = __builtin_fma(kC0, r, kC1);
+  const double y = __builtin_fma(z, r * r, __builtin_fma(kC2, r, 1.0));
+#else
+  const double r = z - kd;
+  z = kC0 * r + kC1;
+  const double y = z * (r * r) + (kC2 * r + 1.0);
+#endif
+  return (float)(y * s);
+}
+
+// exp of a binary32 value, bit-identical to glibc 2.35's expf.
+LLMHIP_HD float glibc_expf_tab(float x, const uint64_t* tab) {
   const uint32_t ux = f32_bits(x);
   const uint32_t abstop = (ux >> 20) & 0x7ff;
   if (abstop >= (f32_bits(88.0f) >> 20)) {
@@ -92,37 +118,7 @@ LLMHIP_HD float glibc_expf_tab(float x, const uint64_t* tab) {
     if (x > 0x1.62e42ep6f) return f32_from_bits(0x7f800000u);  // overflow
     if (x < -0x1.9fe368p6f) return 0.0f;                         // underflow
   }
-  const double xd = (double)x;
-#if LLMHIP_EXPF_FUSED
-  double kd = __builtin_fma(kInvLn2N, xd, kShift);
-  const uint64_t ki = f64_bits(kd);
-  kd -= kShift;
-  const double r = __builtin_fma(kInvLn2N, xd, -kd);
-  uint64_t t = tab[ki % 32];
-  t += ki << 47;
-  const double s = f64_from_bits(t);
-  const double z = __builtin_fma(kC0, r, kC1);
-  const double r2 = r * r;
-  double y = __builtin_fma(kC2, r, 1.0);
-  y = __builtin_fma(z, r2, y);
-  y = y * s;
-  return (float)y;
-#else
-  double z = kInvLn2N * xd;
-  double kd = z + kShift;
-  const uint64_t ki = f64_bits(kd);
-  kd -= kShift;
-  const double r = z - kd;
-  uint64_t t = tab[ki % 32];
-  t += ki << 47;
-  const double s = f64_from_bits(t);
-  z = kC0 * r + kC1;
-  const double r2 = r * r;
-  double y = kC2 * r + 1.0;
-  y = z * r2 + y;
-  y = y * s;
-  return (float)y;
-#endif
+  return glibc_expf_mid(x, tab);
 }
 
 #if !defined(__HIPCC__)

@@ -460,27 +460,9 @@ struct ListSrc {
   }
 };
 
-// glibc_expf_tab's steps for kExactMin <= y <= 0, without its tests for the
-// ends of the range: the same value, in binary64 (which gfx950 runs at the
-// vector ALU's binary32 rate).
+// Terms at or above kExactMin take glibc_expf_mid (binary64, which gfx950 runs
+// at the vector ALU's binary32 rate) and a multiplication by 1 / S.
 constexpr float kExactMin = -60.0f;
-__device__ __forceinline__ float exact_x(float y, const uint64_t* tab) {
-  const double kInvLn2N = 0x1.71547652b82fep+0 * 32.0;
-  const double kShift = 0x1.8p+52;
-  const double kC0 = 0x1.c6af84b912394p-5 / (32.0 * 32.0 * 32.0);
-  const double kC1 = 0x1.ebfce50fac4f3p-3 / (32.0 * 32.0);
-  const double kC2 = 0x1.62e42ff0c52d6p-1 / 32.0;
-  const double yd = (double)y;
-  double kd = __builtin_fma(kInvLn2N, yd, kShift);
-  const uint32_t ki = (uint32_t)f64_bits(kd);
-  kd -= kShift;
-  const double r = __builtin_fma(kInvLn2N, yd, -kd);
-  const uint64_t e = tab[ki % 32u];  // + ki << 47, which reaches the upper word only
-  const double s = f64_from_bits(((uint64_t)((uint32_t)(e >> 32) + (ki << 15)) << 32) | (uint32_t)e);
-  const double z = __builtin_fma(kC0, r, kC1);
-  const double p = __builtin_fma(z, r * r, __builtin_fma(kC2, r, 1.0));
-  return (float)(p * s);
-}
 
 // One or two folds over the row's terms in sorted order (see the file
 // comment). Two folds (the top-p cumulative and the walk, which take the same
@@ -737,7 +719,7 @@ __device__ __forceinline__ bool run_folds(FoldSpec (&fs)[NF], float mx, float u,
     const uint32_t bi = L.binfo[k];
     float t;
     if (__builtin_expect(y >= kExactMin, 1)) {
-      t = exact_x(y, L.exptab);
+      t = glibc_expf_mid(y, L.exptab);
       if constexpr (NF == 2) t = (float)((double)t * rcpS);
     } else {
       t = term_of(glibc_expf_tab(y, L.exptab));

@@ -28,13 +28,14 @@ SRC = textwrap.dedent(r"""
     int main(int argc, char** argv) {
       const uint64_t lo = strtoull(argv[1], 0, 0), hi = strtoull(argv[2], 0, 0);
       std::atomic<unsigned long long> bad{0};
+      const bool mid = argc > 3;
       const int nt = 8;
       std::vector<std::thread> th;
       for (int t = 0; t < nt; ++t) th.emplace_back([&, t] {
         unsigned long long b = 0;
         for (uint64_t u = lo + t; u < hi; u += nt) {
           const float x = llmhip::f32_from_bits((uint32_t)u);
-          const float a = expf(x), c = llmhip::glibc_expf(x);
+          const float a = mid ? llmhip::glibc_expf_mid(x, llmhip::kExp2fTab) : expf(x), c = llmhip::glibc_expf(x);
           if (llmhip::f32_bits(a) != llmhip::f32_bits(c) && !(isnan(a) && isnan(c))) ++b;
         }
         bad += b;
@@ -57,8 +58,8 @@ def _build(tmp_path, fused: int) -> Path:
     return exe
 
 
-def _mismatches(exe, lo, hi) -> int:
-    out = subprocess.run([str(exe), hex(lo), hex(hi)], check=True, capture_output=True, text=True)
+def _mismatches(exe, lo, hi, *mid) -> int:
+    out = subprocess.run([str(exe), hex(lo), hex(hi), *mid], check=True, capture_output=True, text=True)
     return int(out.stdout.strip())
 
 
@@ -72,3 +73,14 @@ def test_unfused_control_variant_differs(tmp_path):
     # exhaustive comparison is sharp enough to see the contraction choice.
     exe = _build(tmp_path, 0)
     assert _mismatches(exe, 0, 1 << 32) > 0
+
+
+@pytest.mark.parametrize("fused", [0, 1])
+def test_the_form_without_range_tests_is_the_same_function(tmp_path, fused):
+    """The full-vocabulary kernel takes its terms for y in [-60, 0] from
+    glibc_expf_mid and recomputes some of them with glibc_expf_tab: both must
+    be one function, whichever variant is built."""
+    exe = _build(tmp_path, fused)
+    zero, minus_60 = 0x80000000, 0xC2700000  # the bits of -0.0 .. -60.0 ascend
+    assert _mismatches(exe, zero, minus_60 + 1, "mid") == 0
+    assert _mismatches(exe, 0, 1, "mid") == 0
