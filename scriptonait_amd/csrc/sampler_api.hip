@@ -31,7 +31,7 @@ hipError_t launch_vocab(const SampleArgs& a, bool plain, hipStream_t s);
 hipError_t launch_seen_bits(const uint32_t* tokens, uint64_t n, uint32_t V, uint32_t* bits, hipStream_t s);
 hipError_t launch_take_status(uint32_t* words, hipStream_t s);
 hipError_t launch_host_status(uint32_t* word, uint32_t* out, hipStream_t s);
-hipError_t launch_stream(const SampleArgs& a, bool bigk, hipStream_t s);
+hipError_t launch_stream(const SampleArgs& a, bool bigk, bool refine, hipStream_t s);
 hipError_t launch_read_floor(const float* logits, uint64_t ld, uint32_t B, uint32_t V, int read, float* out,
                              hipStream_t s);
 hipError_t launch_tied_head(const float* hidden, uint64_t ldh, const float* embed, uint64_t lde, float* logits,
@@ -226,6 +226,7 @@ int enqueue(llmhip_ctx* ctx, const float* logits, size_t B, size_t V, size_t ld,
   }
   uint32_t classes = 0;
   bool bigk = false;  // some top-k row has K > 64, or more to list than the small-K kernels rank
+  bool refine = false;  // some row of the streaming path raises its threshold
   bool penalized = false;  // some row has a repetition penalty (and the call a history)
   uint32_t row_cls[128] = {};  // each row's class index (SampleArgs::row_cls), for calls of <= kRowClsRows rows
   for (size_t b = 0; b < (params_stride ? B : 1); ++b) {
@@ -233,6 +234,7 @@ int enqueue(llmhip_ctx* ctx, const float* logits, size_t B, size_t V, size_t ld,
     const uint32_t c = route_class(p, (uint32_t)V);
     classes |= c;
     bigk = bigk || (c == kClassTopK && (p.top_k > 64u || (V > kMaxFastV && stream_bigk(p.top_k, (uint32_t)V))));
+    refine = refine || (c == kClassTopK && V > kMaxFastV && stream_refines(p.top_k, (uint32_t)V));
     penalized = penalized || p.repetition_penalty != 1.0f;
     if (b < kRowClsRows) row_cls[b >> 4] |= (uint32_t)__builtin_ctz(c) << ((b & 15u) * 2u);
   }
@@ -306,7 +308,7 @@ int enqueue(llmhip_ctx* ctx, const float* logits, size_t B, size_t V, size_t ld,
   }
   if (stream_mask) {
     a.row_class_mask = stream_mask;
-    HIP_TRY(launch_stream(a, bigk, s));
+    HIP_TRY(launch_stream(a, bigk, refine, s));
   }
   if (vocab_mask) {
     a.row_class_mask = vocab_mask;

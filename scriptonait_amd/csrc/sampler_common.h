@@ -367,20 +367,33 @@ __host__ __device__ __forceinline__ uint32_t row_class(const llmhip_params& p, u
 // The streaming path (top-k rows past kMaxFastV) lists about 1.2 K values
 // per 32768 of the row (its threshold comes from the row's first 32768
 // values) in a list of kStreamCand. Where that does not fit with a margin, or
-// K is above 256, it raises the threshold after each 32768 values: part j then
-// lists about K / j, and the first at most 1.45 K (the first threshold is the
-// lower edge of a bin 1/8 of a value wide). It takes a row when either fits,
-// and when the penalty is at least 1 (one below 1 can raise a value past the
-// threshold).
+// where it is faster (stream_refines), it raises the threshold after each 32768
+// values: part j then lists about K / j, and the first at most 1.45 K (the first
+// threshold is the lower edge of a bin 1/8 of a value wide). It takes a row when
+// either fits, and when the penalty is at least 1 (one below 1 can raise a value
+// past the threshold).
 constexpr uint32_t kStreamSpan = 32768;
 constexpr uint32_t kStreamCand = 4096;
-__host__ __device__ __forceinline__ uint32_t stream_parts(uint32_t V) { return (V + kStreamSpan - 1u) / kStreamSpan; }
-__host__ __device__ __forceinline__ bool stream_fits(uint32_t K, uint32_t V) {
+__host__ __device__ constexpr uint32_t stream_parts(uint32_t V) { return (V + kStreamSpan - 1u) / kStreamSpan; }
+__host__ __device__ constexpr bool stream_fits(uint32_t K, uint32_t V) {
   return (uint64_t)K * stream_parts(V) * 5u <= (uint64_t)kStreamCand * 4u;
 }
-__host__ __device__ __forceinline__ bool stream_refines(uint32_t K, uint32_t V) {
-  return K > 256u || !stream_fits(K, V);
+// Raising the threshold costs a histogram and a selection per 32768 values, and
+// saves listing and sorting what later parts hold above the first threshold: it
+// pays past one and a half parts and for K in the hundreds. 512 rows, us without
+// and with: V = 33000 K = 257 51.2 / 56.9, K = 1000 82.9 / 86.0; V = 40000 K = 600
+// 68.3 / 72.3; V = 50260 K = 300 57.7 / 60.1, K = 400 66.6 / 64.1, K = 1000 90.5 /
+// 87.5; V = 65536 K = 300 62.3 / 62.3, K = 400 71.1 / 66.7; V = 81920 K = 257 68.9 /
+// 67.4; V = 131072 K = 257 89.9 / 82.2.
+__host__ __device__ constexpr bool stream_refines(uint32_t K, uint32_t V) {
+  if (!stream_fits(K, V)) return true;
+  return V > 2u * kStreamSpan ? K > 256u : V >= kStreamSpan + kStreamSpan / 2u && K > 320u;
 }
+static_assert(!stream_refines(257u, 33000u) && !stream_refines(1567u, 49151u) && !stream_refines(320u, 65536u),
+              "slower there");
+static_assert(stream_refines(400u, 50260u) && stream_refines(257u, 65537u) && stream_refines(820u, 131072u) &&
+                  stream_refines(60u, 8388608u),
+              "faster there, or would not fit");
 // Rows of K <= 64 that the streaming kernel compiled for them may hand over
 // (it ranks 512 listed values, of about 1.25 K per part).
 __host__ __device__ __forceinline__ bool stream_bigk(uint32_t K, uint32_t V) {

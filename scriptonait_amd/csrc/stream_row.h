@@ -143,9 +143,12 @@ __device__ __forceinline__ void stream_load(float (&buf)[kSNS * 4], const float*
 // (a ring, maybe a count table); the other calls run a variant compiled without
 // that code, whose loop keeps fewer values live. BIGK: some row of the launch
 // has K > 64; without it the kernel holds only the register rank and tail, and
-// a row listing more than 512 values is handed over.
-template <bool TAIL, bool FULL, bool BIGK>
+// a row listing more than 512 values is handed over. REFINE: some row raises its
+// threshold (one kernel for both cost the rows that do not 1 to 3 us: 512 rows of
+// 33000 at K = 100 41.5 -> 42.5 us, of 131072 75.0 -> 78.0).
+template <bool TAIL, bool FULL, bool BIGK, bool REFINE>
 __device__ __forceinline__ void stream_rows(const SampleArgs& a, StreamKernelLds& U) {
+  static_assert(BIGK || !REFINE, "rows that raise their threshold list more than 512 values");
   StreamLds& L = U.s;
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
@@ -226,7 +229,7 @@ __device__ __forceinline__ void stream_rows(const SampleArgs& a, StreamKernelLds
     }
     const bool use_pen = rp != 1.0f && hr.H > 0u;
     // Rows of a large K raise the threshold as they stream (below).
-    const bool refine = BIGK && stream_refines(K, V);
+    const bool refine = REFINE && stream_refines(K, V);
     uint32_t* listed = reinterpret_cast<uint32_t*>(L.tmp);  // their histogram (the sort's buffer, free until then)
 
     if (outcome == 0u) {

@@ -3,6 +3,6 @@
 
 namespace llmhip {
 
-template hipError_t launch_stream_k<true>(const SampleArgs&, hipStream_t);
+template hipError_t launch_stream_k<true, false>(const SampleArgs&, hipStream_t);
 
 }  // namespace llmhip

@@ -176,14 +176,15 @@ def test_full_batches_at_small_k(sampler, cfg, k):
     assert g["handovers"] == 0
 
 
-# Rows whose K is above 256, or whose list would not hold 1.2 K values per
-# 32768, raise the threshold as they stream: both sides of K = 256 and of the
-# largest K taken (1169 at four parts, 940 at eight), the smallest vocabulary
-# and ragged ones. shape: normal, heavy-tailed, ascending (every part's values
+# Rows whose list would not hold 1.2 K values per 32768, and rows of a large K
+# past one and a half parts, raise the threshold as they stream: both sides of
+# that rule (stream_refines) and of the largest K taken (1169 at four parts,
+# 940 at eight), the smallest vocabulary and ragged ones. shape: normal, heavy-tailed, ascending (every part's values
 # above the last one's: the threshold rises with each), or few distinct values.
 @pytest.mark.parametrize("V,K,shape,handed", [
     (32769, 257, "normal", 0), (32769, 1567, "normal", 0), (50257, 1000, "normal", 0), (65537, 900, "gumbel", 0),
-    (98304, 1169, "gumbel", 0), (131072, 256, "normal", 0), (131072, 257, "gumbel", 0), (131072, 820, "normal", 0),
+    (49151, 1567, "normal", 0), (49152, 320, "normal", 0), (49152, 321, "normal", 0), (65536, 1567, "normal", 0),
+    (65537, 256, "normal", 0), (65537, 257, "normal", 0), (98304, 1169, "gumbel", 0), (131072, 256, "normal", 0), (131072, 257, "gumbel", 0), (131072, 820, "normal", 0),
     (131072, 1169, "normal", 0), (131072, 1170, "normal", 0), (131071, 1000, "gumbel", 0), (262147, 940, "normal", 0),
     (400001, 60, "normal", 0), (131072, 300, "ascending", None), (131072, 700, "coarse", None)])
 @pytest.mark.parametrize("extra", ["plain", "history", "mask"])
