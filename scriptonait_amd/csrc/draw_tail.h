@@ -46,8 +46,14 @@ __device__ __forceinline__ void stage_exp_terms(float* buf, uint32_t n, KeyAt ke
 // tested (c never decreases; r - p < 0 exactly when r < p), the block that
 // decides being resolved once, one lane per term. Terms past the kept
 // prefix are set to +0.0, which leaves either fold unchanged.
+// AHEAD: each block's terms are read while the one before it is folded. That
+// pays on the register path (256 rows of 32000: 64.1 -> 63.5 us at K = 2000,
+// 101.5 -> 100.2 at 4000) and for the large K of the streaming kernels that
+// raise their threshold (512 rows of 131072, K = 1000: 110.6 -> 109.4). In the
+// other streaming kernels, which have no register left for it, it does not (512
+// rows of 33000: 41.4 -> 42.2 us at K = 100, 48.0 -> 48.7 at 200).
 // Must be called by all 64 lanes of exactly one wave.
-template <bool STAGED = false, class KeyAt, class IdAt>
+template <bool STAGED = false, bool AHEAD = false, class KeyAt, class IdAt>
 __device__ __forceinline__ void draw_tail_lds(const SampleArgs& a, uint32_t b, uint32_t len_b, const llmhip_params& P,
                                               uint32_t n, KeyAt key_at, IdAt id_at, uint64_t st, const uint64_t* tab,
                                               float* buf) {
@@ -90,14 +96,11 @@ __device__ __forceinline__ void draw_tail_lds(const SampleArgs& a, uint32_t b, u
   // no such tie whose counts keep S in its binade adds their total at once
   // (exact: S / u + total < 2^24); any other block (a binade change, a tie, a
   // term or sum that is not finite) is added term by term.
-  // Each block's terms are read while the one before it is folded, here and
-  // in the two folds below (256 rows of 32000: 64.1 -> 63.5 us at K = 2000,
-  // 101.5 -> 100.2 at 4000).
   add_terms(0u, min(nr, 64u) / 4u);
-  float tnext = nr > 64u ? buf[64u + lane] : 0.0f;
+  float tnext = AHEAD && nr > 64u ? buf[64u + lane] : 0.0f;
   for (uint32_t base = 64u; base < nr; base += 64u) {
-    const float t = tnext;
-    if (base + 64u < nr) tnext = buf[base + 64u + lane];
+    const float t = AHEAD ? tnext : buf[base + lane];
+    if (AHEAD && base + 64u < nr) tnext = buf[base + 64u + lane];
     bool step = !(sum >= 1.0f) || !isfinite(sum);
     if (!step) {
       const int E = (int)((__float_as_uint(sum) >> 23) & 0xffu) - 127;  // sum is normal, >= 1
@@ -126,11 +129,11 @@ __device__ __forceinline__ void draw_tail_lds(const SampleArgs& a, uint32_t b, u
   uint32_t keep = n;
   if (P.min_p > 0.0f) {
     const float thr = P.min_p * (buf[0] / sum);
-    float enext = buf[lane];
+    float enext = AHEAD ? buf[lane] : 0.0f;
     for (uint32_t c = 0; c < n; c += 64u) {
       const uint32_t i = c + lane;
-      const float p = enext / sum;
-      if (c + 64u < n) enext = buf[i + 64u];  // (staged to a multiple of 64)
+      const float p = (AHEAD ? enext : buf[i]) / sum;  // (staged to a multiple of 64)
+      if (AHEAD && c + 64u < n) enext = buf[i + 64u];
       if (i < n) buf[i] = p;
       const uint64_t fail = __ballot(i < n && !(p >= thr));
       if (fail) {
@@ -206,10 +209,10 @@ __device__ __forceinline__ void draw_tail_lds(const SampleArgs& a, uint32_t b, u
       }
     };
     const uint32_t kr = (keep + 63u) & ~63u;
-    float pnext = buf[lane];
+    float pnext = AHEAD ? buf[lane] : 0.0f;
     for (uint32_t b0 = 0u; b0 < kr && !done; b0 += 64u) {
-      const float pj = pnext;  // 0 past keep
-      if (b0 + 64u < kr) pnext = buf[b0 + 64u + lane];
+      const float pj = AHEAD ? pnext : buf[b0 + lane];  // 0 past keep
+      if (AHEAD && b0 + 64u < kr) pnext = buf[b0 + 64u + lane];
       // The first block term by term (c starts at 0 and climbs through
       // binades), and a block with few kept terms left (a scan costs about
       // as much as 30 steps).
@@ -297,10 +300,10 @@ __device__ __forceinline__ void draw_tail_lds(const SampleArgs& a, uint32_t b, u
       }
     };
     const uint32_t sr = (stop + 63u) & ~63u;
-    float pnext = buf[lane];
+    float pnext = AHEAD ? buf[lane] : 0.0f;
     for (uint32_t b0 = 0u; b0 < sr && !found; b0 += 64u) {
-      const float pj = pnext;  // 0 past stop
-      if (b0 + 64u < sr) pnext = buf[b0 + 64u + lane];
+      const float pj = AHEAD ? pnext : buf[b0 + lane];  // 0 past stop
+      if (AHEAD && b0 + 64u < sr) pnext = buf[b0 + 64u + lane];
       // Term by term: the first block of a short walk (it usually ends
       // there), and a block with few terms left.
       bool step = (b0 == 0u && stop <= 256u) || stop - b0 < 32u || !(r >= 0x1p-126f) || !isfinite(r);

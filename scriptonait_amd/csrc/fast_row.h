@@ -1416,7 +1416,7 @@ __device__ __forceinline__ bool fast_row(const SampleArgs& a, FastLds<NCH, BIGK>
       lds_barrier();
       LLMHIP_MARK(7);
       if (wave == 0)
-        draw_tail_lds<true>(a, b, len_b, P, K, key_at, [&](uint32_t i) { return ~(uint32_t)srt[i]; }, rng0, L.exptab,
+        draw_tail_lds<true, true>(a, b, len_b, P, K, key_at, [&](uint32_t i) { return ~(uint32_t)srt[i]; }, rng0, L.exptab,
                             buf);
       LLMHIP_MARK(8);
       return true;
@@ -1449,7 +1449,7 @@ __device__ __forceinline__ bool fast_row(const SampleArgs& a, FastLds<NCH, BIGK>
       draw_tail_bcast(a, b, len_b, P, K, lane < K ? L.skey[lane] : kKeyNone, lane < K ? L.sid[lane] : 0u,
                       u_draw, st_next, L.exptab, L.tail);
     } else {
-      draw_tail_lds<true>(a, b, len_b, P, K, [&](uint32_t i) { return L.skey[i]; },
+      draw_tail_lds<true, true>(a, b, len_b, P, K, [&](uint32_t i) { return L.skey[i]; },
                           [&](uint32_t i) { return L.sid[i]; }, rng0, L.exptab, reinterpret_cast<float*>(L.ord));
     }
   }

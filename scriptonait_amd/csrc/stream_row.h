@@ -544,7 +544,7 @@ __device__ __forceinline__ void stream_rows(const SampleArgs& a, StreamKernelLds
         auto id_at = [&](uint32_t i) { return ~(uint32_t)srt[i]; };
         stage_exp_terms(buf, K, key_at, L.exptab, tid, kBlock);
         lds_barrier();
-        if (wave == 0) draw_tail_lds<true>(a, b, len_b, P, K, key_at, id_at, rng0, L.exptab, buf);
+        if (wave == 0) draw_tail_lds<true, REFINE>(a, b, len_b, P, K, key_at, id_at, rng0, L.exptab, buf);
       }
     }
     if (jn >= nrows) break;
