@@ -719,7 +719,7 @@ __device__ __forceinline__ bool run_folds(FoldSpec (&fs)[NF], float mx, float u,
     const uint32_t bi = L.binfo[k];
     float t;
     if (__builtin_expect(y >= kExactMin, 1)) {
-      t = glibc_expf_mid(y, L.exptab);
+      t = glibc_expf_mid<true>(y, L.exptab);
       if constexpr (NF == 2) t = (float)((double)t * rcpS);
     } else {
       t = term_of(glibc_expf_tab(y, L.exptab));

@@ -35,7 +35,7 @@ SRC = textwrap.dedent(r"""
         unsigned long long b = 0;
         for (uint64_t u = lo + t; u < hi; u += nt) {
           const float x = llmhip::f32_from_bits((uint32_t)u);
-          const float a = mid ? llmhip::glibc_expf_mid(x, llmhip::kExp2fTab) : expf(x), c = llmhip::glibc_expf(x);
+          const float a = mid ? llmhip::glibc_expf_mid<true>(x, llmhip::kExp2fTab) : expf(x), c = llmhip::glibc_expf(x);
           if (llmhip::f32_bits(a) != llmhip::f32_bits(c) && !(isnan(a) && isnan(c))) ++b;
         }
         bad += b;
