@@ -69,6 +69,7 @@ constexpr uint32_t kSPend = 512;             // listed values waiting for their 
 
 // misc[] slots
 enum : uint32_t { kSCandN = 0, kSDistinct = 1, kSFull = 2, kSPendN = 3, kSTau = 4, kSMisc = 5 };
+constexpr uint32_t kSDrop = 3072;    // listed values from which those below a raised threshold are dropped
 constexpr uint32_t kSRefShift = 14;  // key bits below a refined threshold's bin (1/512 of a value)
 
 struct StreamLds {
@@ -339,6 +340,7 @@ __device__ __forceinline__ void stream_rows(const SampleArgs& a, StreamKernelLds
       // the value picked out of the buffer by selects (a register array
       // takes constant indices only).
       uint32_t o = base + inc - hc;
+      const bool counted = refine && base < kSCand;  // (a row whose list is full is handed over)
       for (uint32_t h = hits; h != 0u; h &= h - 1u) {
         const uint32_t e = (uint32_t)__builtin_ctz(h);
         float v = buf[0];
@@ -347,7 +349,7 @@ __device__ __forceinline__ void stream_rows(const SampleArgs& a, StreamKernelLds
         const uint32_t i = 4u * (p * kSPieceQ + (e >> 2) * kBlock + tid) + (e & 3u);
         if (o < kSCand) L.list[o] = ((uint64_t)__float_as_uint(v) << 32) | i;
         ++o;
-        if (refine) atomicAdd(&listed[min((f2key(v) - tkey) >> kSRefShift, kFineBins - 1u)], 1u);
+        if (counted) atomicAdd(&listed[min((f2key(v) - tkey) >> kSRefShift, kFineBins - 1u)], 1u);
       }
       // Marked values wait in their own list: their penalty is applied once
       // the row is streamed (a penalty loop here would weigh on every
@@ -428,8 +430,41 @@ __device__ __forceinline__ void stream_rows(const SampleArgs& a, StreamKernelLds
               if (lane == 0) L.misc[kSTau] = t;
               __builtin_amdgcn_s_setprio(0);
             }
+            const uint32_t nl = L.misc[kSCandN];  // (nothing is listed until the next barrier)
             lds_barrier();
             tf = fmaxf(tf, key2f(max(L.misc[kSTau], tkey)));
+            if (nl > kSCand) {
+              // A list that has overflowed (values that grow along the row): the
+              // rest of the row is read but not listed. (Leaving the loop here
+              // cost every row 5%.)
+              tf = INFINITY;
+            } else if (nl > kSDrop || p + 2u >= np) {
+              // The listed values below the threshold are dropped: at the row's
+              // end (the others are sorted), and from a list that the parts still
+              // to come could overflow (ties at the threshold).
+              static_assert(kSCand == 4u * kBlock, "four per thread");
+              uint64_t r[4];
+              bool in[4];
+#pragma unroll
+              for (uint32_t q = 0; q < 4u; ++q) {
+                const uint32_t i = tid + q * kBlock;
+                r[q] = i < nl ? L.list[i] : 0ull;
+                in[q] = i < nl && __uint_as_float((uint32_t)(r[q] >> 32)) >= tf;
+              }
+              lds_barrier();
+              if (tid == 0) L.misc[kSCandN] = 0u;
+              lds_barrier();
+#pragma unroll
+              for (uint32_t q = 0; q < 4u; ++q) {
+                const uint64_t m = __ballot(in[q]);
+                if (m == 0ull) continue;
+                uint32_t o = 0u;
+                if (lane == 0) o = atomicAdd(&L.misc[kSCandN], (uint32_t)__popcll((unsigned long long)m));
+                o = readlane_u32(o, 0) + lanes_below(m);
+                if (in[q]) L.list[o] = r[q];
+              }
+              lds_barrier();
+            }
           }
         }
         fetched = true;
@@ -450,32 +485,6 @@ __device__ __forceinline__ void stream_rows(const SampleArgs& a, StreamKernelLds
         }
         LLMHIP_MARK(5);
         lds_barrier();
-        if (refine && L.misc[kSCandN] <= kSCand) {
-          // Only the listed values at or above the last threshold are sorted.
-          static_assert(kSCand == 4u * kBlock, "four per thread");
-          const uint32_t n0 = L.misc[kSCandN];
-          uint64_t r[4];
-          bool in[4];
-#pragma unroll
-          for (uint32_t q = 0; q < 4u; ++q) {
-            const uint32_t i = tid + q * kBlock;
-            r[q] = i < n0 ? L.list[i] : 0ull;
-            in[q] = i < n0 && __uint_as_float((uint32_t)(r[q] >> 32)) >= tf;
-          }
-          lds_barrier();
-          if (tid == 0) L.misc[kSCandN] = 0u;
-          lds_barrier();
-#pragma unroll
-          for (uint32_t q = 0; q < 4u; ++q) {
-            const uint64_t m = __ballot(in[q]);
-            if (m == 0ull) continue;
-            uint32_t o = 0u;
-            if (lane == 0) o = atomicAdd(&L.misc[kSCandN], (uint32_t)__popcll((unsigned long long)m));
-            o = readlane_u32(o, 0) + lanes_below(m);
-            if (in[q]) L.list[o] = r[q];
-          }
-          lds_barrier();
-        }
         // The marked values' penalties (generate.rs:343-352), stopping once
         // a value is below the threshold (exact for rp >= 1).
         const uint32_t npend = L.misc[kSPendN];

@@ -179,14 +179,18 @@ def test_full_batches_at_small_k(sampler, cfg, k):
 # Rows whose list would not hold 1.2 K values per 32768, and rows of a large K
 # past one and a half parts, raise the threshold as they stream: both sides of
 # that rule (stream_refines) and of the largest K taken (1169 at four parts,
-# 940 at eight), the smallest vocabulary and ragged ones. shape: normal, heavy-tailed, ascending (every part's values
-# above the last one's: the threshold rises with each), or few distinct values.
+# 940 at eight), the smallest vocabulary and ragged ones. shape: normal,
+# heavy-tailed, ascending (every part's values above the last one's: the
+# threshold rises with each), few distinct values (ties that fill the list unless
+# those below the threshold are dropped on the way), or sorted (the second part
+# overflows the list, and the rest is not listed).
 @pytest.mark.parametrize("V,K,shape,handed", [
     (32769, 257, "normal", 0), (32769, 1567, "normal", 0), (50257, 1000, "normal", 0), (65537, 900, "gumbel", 0),
     (49151, 1567, "normal", 0), (49152, 320, "normal", 0), (49152, 321, "normal", 0), (65536, 1567, "normal", 0),
     (65537, 256, "normal", 0), (65537, 257, "normal", 0), (98304, 1169, "gumbel", 0), (131072, 256, "normal", 0), (131072, 257, "gumbel", 0), (131072, 820, "normal", 0),
     (131072, 1169, "normal", 0), (131072, 1170, "normal", 0), (131071, 1000, "gumbel", 0), (262147, 940, "normal", 0),
-    (400001, 60, "normal", 0), (131072, 300, "ascending", None), (131072, 700, "coarse", None)])
+    (400001, 60, "normal", 0), (131072, 300, "ascending", None), (131072, 700, "coarse", None),
+    (131072, 1000, "coarse", 0), (98303, 1100, "coarse", 0), (131072, 1000, "sorted", 4), (98304, 500, "sorted", 4)])
 @pytest.mark.parametrize("extra", ["plain", "history", "mask"])
 def test_threshold_raised_while_streaming(sampler, V, K, shape, handed, extra):
     rs = np.random.default_rng(V + K)
@@ -194,6 +198,8 @@ def test_threshold_raised_while_streaming(sampler, V, K, shape, handed, extra):
     x = rs.standard_normal((B, V)) if shape != "gumbel" else rs.gumbel(size=(B, V))
     if shape == "ascending":
         x = x + 6.0 * np.arange(V) / V
+    if shape == "sorted":
+        x = np.sort(x, axis=1)
     if shape == "coarse":
         x = np.round(x * 4.0) / 4.0
     w = make_workload(5, B=B, V=64)
