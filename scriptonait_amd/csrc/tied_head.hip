@@ -12,12 +12,14 @@
 // accumulating in the matrix cores; every product is rounded on its own and
 // every accumulator takes its additions one at a time.
 //
-// Three kernels share this file (launch_tied_head picks one):
+// Four kernels share this file (launch_tied_head picks one):
 //
 //  * tied_head_mfma_kernel: the matrix cores make the products and the
 //    vector ALUs only add them, in 32 x 32 tiles per wave.
 //  * tied_head_mfma16_kernel: the same in 16 x 16 tiles, for few rows or
 //    few tiles.
+//  * tied_head_valu_kernel: vector multiplies and adds, for short rows (h up
+//    to 64), where the logits' writes and the workgroups' latency are the time.
 //  * tied_head_gemv_kernel (one to four rows): one pass over embed with no
 //    padding rows, bound by reading embed.
 #include <hip/hip_runtime.h>
@@ -311,6 +313,78 @@ __global__ __launch_bounds__(kHeadThreads, 4) void tied_head_mfma16_kernel(HeadA
 }
 
 // ---------------------------------------------------------------------------
+// Short rows: vector multiplies and adds. A workgroup computes 32 rows x 128
+// outputs, thread (tr, to) of its 8 x 32 threads rows tr + 8i and outputs to +
+// 32j, 64 accumulators in registers. The shared dimension is staged 16 floats
+// at a time with no load in flight behind the products, so it loses where h is
+// long; where h is short its small prologue and its writes, consecutive
+// workgroups filling consecutive parts of the same rows, win. B = 256, h = 32:
+// V = 32000 28.3 us with the sampler (34.5 with 32 x 32 tiles, 32.5 with 16 x
+// 16), V = 65536 51.5 (65.5, 62.3); h = 16: 24.4 (34.9, 33.3).
+// ---------------------------------------------------------------------------
+constexpr uint32_t kValuRows = 32, kValuOuts = 128, kValuStage = 4;  // chunks per stage
+
+__global__ __launch_bounds__(kHeadThreads) void tied_head_valu_kernel(HeadArgs a) {
+  __shared__ f4 xs[kValuStage][kValuRows];
+  __shared__ f4 ws[kValuStage][kValuOuts];
+  const uint32_t t = threadIdx.x, tr = t >> 5, to = t & 31u;
+  const uint32_t o0 = a.out0 + (blockIdx.x % a.out_tiles) * kValuOuts;
+  const uint32_t r0 = a.row0 + (blockIdx.x / a.out_tiles) * kValuRows;
+  const uint32_t nch = a.h >> 2;
+
+  f4 acc[4][4];  // [row i][output j], element k: accumulator k
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+
+  // Staging: thread t loads chunk t & 3 of embed rows t >> 2 and 64 further,
+  // and below 128 of hidden row t >> 2. Rows past the last read the last
+  // (their results are not stored).
+  const uint32_t sq = t & 3u, sr = t >> 2;
+  const float* xrow = a.hidden + (size_t)min(r0 + (sr & 31u), a.B - 1u) * a.ldh;
+  const float* wrow0 = a.embed + (size_t)min(o0 + sr, a.V - 1u) * a.lde;
+  const float* wrow1 = a.embed + (size_t)min(o0 + 64u + sr, a.V - 1u) * a.lde;
+  for (uint32_t c0 = 0; c0 < nch; c0 += kValuStage) {
+    const f4 xv = head_chunk(xrow, c0 + sq, nch);
+    const f4 wv0 = head_chunk(wrow0, c0 + sq, nch), wv1 = head_chunk(wrow1, c0 + sq, nch);
+    __syncthreads();  // the previous stage's reads are done
+    if (t < 128u) xs[sq][sr] = xv;
+    ws[sq][sr] = wv0;
+    ws[sq][64u + sr] = wv1;
+    __syncthreads();
+#pragma unroll
+    for (uint32_t c = 0; c < kValuStage; ++c) {
+      f4 x[4], w[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        x[i] = xs[c][tr + 8u * i];
+        w[i] = ws[c][to + 32u * i];
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int k = 0; k < 4; ++k) acc[i][j][k] = acc[i][j][k] + x[i][k] * w[j][k];
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t row = r0 + tr + 8u * i;
+    if (row >= a.B) continue;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t out = o0 + to + 32u * j;
+      if (out >= a.V) continue;
+      const float s = (acc[i][j][0] + acc[i][j][1]) + (acc[i][j][2] + acc[i][j][3]);
+      a.logits[(size_t)row * a.ldl + out] =
+          s + head_tail(a.hidden + (size_t)row * a.ldh, a.embed + (size_t)out * a.lde, a.h);
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Few rows: one pass over embed. A wave takes 16 outputs; lanes 4i .. 4i+3
 // share output i, lane j of the four holding its accumulator j for all R
 // rows. They load 4 consecutive chunks of the row at a time (64 bytes, a
@@ -437,32 +511,44 @@ hipError_t launch_gemv(const HeadArgs& a0, hipStream_t s) {
   return hipSuccess;
 }
 
-// TILE x TILE results per wave, WR x WO waves.
-template <int TILE, int WR, int WO>
-hipError_t launch_mfma(const HeadArgs& a0, hipStream_t s) {
+// Launches over slices of at most 2^10 row tiles x 2^12 output tiles.
+template <class Launch>
+hipError_t launch_slices(const HeadArgs& a0, uint32_t rows, uint32_t outs, Launch&& launch) {
   HeadArgs a = a0;
-  constexpr uint32_t kRows = TILE * WR, kOuts = TILE * WO;
-  // Slices of at most 2^10 row tiles x 2^12 output tiles a launch.
   constexpr uint32_t kMaxRowTiles = 1u << 10, kMaxOutTiles = 1u << 12;
-  const uint32_t rts = (a.B + kRows - 1u) / kRows, ots = (a.V + kOuts - 1u) / kOuts;
+  const uint32_t rts = (a.B + rows - 1u) / rows, ots = (a.V + outs - 1u) / outs;
   for (uint32_t t0 = 0; t0 < rts; t0 += kMaxRowTiles) {
-    a.row0 = t0 * kRows;
+    a.row0 = t0 * rows;
     a.row_tiles = std::min(kMaxRowTiles, rts - t0);
     for (uint32_t u0 = 0; u0 < ots; u0 += kMaxOutTiles) {
-      a.out0 = u0 * kOuts;
+      a.out0 = u0 * outs;
       a.out_tiles = std::min(kMaxOutTiles, ots - u0);
-      const uint32_t grid = (a.out_tiles + 7u) / 8u * 8u * a.row_tiles;
-      if constexpr (TILE == 16) {
-        hipLaunchKernelGGL((tied_head_mfma16_kernel<WR, WO>), dim3(grid), dim3(kHeadThreads), 0, s, a);
-      } else {
-        static_assert(TILE == 32 && WR == 2 && WO == 2, "the 32 x 32 kernel's workgroup");
-        hipLaunchKernelGGL(tied_head_mfma_kernel, dim3(grid), dim3(kHeadThreads), 0, s, a);
-      }
+      launch(a);
       const hipError_t e = hipGetLastError();
       if (e != hipSuccess) return e;
     }
   }
   return hipSuccess;
+}
+
+// TILE x TILE results per wave, WR x WO waves.
+template <int TILE, int WR, int WO>
+hipError_t launch_mfma(const HeadArgs& a0, hipStream_t s) {
+  return launch_slices(a0, TILE * WR, TILE * WO, [&](const HeadArgs& a) {
+    const uint32_t grid = (a.out_tiles + 7u) / 8u * 8u * a.row_tiles;
+    if constexpr (TILE == 16) {
+      hipLaunchKernelGGL((tied_head_mfma16_kernel<WR, WO>), dim3(grid), dim3(kHeadThreads), 0, s, a);
+    } else {
+      static_assert(TILE == 32 && WR == 2 && WO == 2, "the 32 x 32 kernel's workgroup");
+      hipLaunchKernelGGL(tied_head_mfma_kernel, dim3(grid), dim3(kHeadThreads), 0, s, a);
+    }
+  });
+}
+
+hipError_t launch_valu(const HeadArgs& a0, hipStream_t s) {
+  return launch_slices(a0, kValuRows, kValuOuts, [&](const HeadArgs& a) {
+    hipLaunchKernelGGL(tied_head_valu_kernel, dim3(a.out_tiles * a.row_tiles), dim3(kHeadThreads), 0, s, a);
+  });
 }
 
 }  // namespace
@@ -478,13 +564,32 @@ hipError_t launch_tied_head(const float* hidden, uint64_t ldh, const float* embe
   if (B == 1) return launch_gemv<1>(a, s);
   if (B == 2) return launch_gemv<2>(a, s);
   if (B <= 4 && V <= 16384) return launch_gemv<4>(a, s);
+  // Short rows and many results: vector multiplies. B x V, us with the sampler,
+  // those and the better matrix-core kernel: h = 16 8 x 65536 24.7 / 25.4, 64 x
+  // 32000 14.2 / 16.2, 512 x 32000 36.4 / 54.3; h = 48 64 x 32000 17.1 / 17.6, 256
+  // x 32000 33.3 / 39.6, but 64 x 8192 13.5 / 11.8 and 32 x 100000 45.0 / 43.7; h =
+  // 64 256 x 65536 71.9 / 76.4, 512 x 32000 68.5 / 68.5, 128 x 32000 25.3 / 25.6,
+  // but 128 x 100000 73.0 / 70.9; h = 96 256 x 65536 94.2 / 94.8, 256 x 32000 50.4
+  // / 48.2.
+  const uint64_t results = (uint64_t)B * V;
+  if (h <= 16u   ? B >= 8u && results >= 1u << 19
+      : h <= 48u ? B >= 64u && results >= 2000000u
+                 : h <= 64u && results >= 16000000u)
+    return launch_valu(a, s);
   // 32 x 32 tiles need two per SIMD to hide their loads (1024 tiles, V =
   // 8192 at 128 rows, h = 256: 17.7 us against 15.0 with 16 x 16 tiles; 2048,
   // at 256 rows: 25.0 against 26.9), and pay for rows padded to 64 (V = 32000,
-  // h = 512: 41.5 us against 37.8 at 48 rows, 42.7 against 44.7 at 64).
+  // h = 512: 41.5 us against 37.8 at 48 rows, 42.7 against 44.7 at 64). Over a
+  // shorter h their prologue counts, the more the more tiles there are. B x V, us
+  // with the sampler, 32 x 32 and 16 x 16: h = 64 256 x 32000 41.0 / 39.1, 512 x
+  // 8192 30.0 / 29.3; h = 96 256 x 8192 19.6 / 20.4, 64 x 50257 39.2 / 35.6, 512 x
+  // 65536 186 / 182; h = 128 256 x 8192 21.5 / 22.3, 256 x 32000 56.0 / 56.4, 128 x
+  // 50257 60.1 / 55.4, 256 x 100000 169 / 165; h = 192 256 x 32000 72.6 / 73.7, 256
+  // x 65536 145 / 147.
   const uint64_t tiles = (uint64_t)((B + 31u) / 32u) * ((V + 31u) / 32u);
   const uint64_t pad64 = ((uint64_t)B + 63u) / 64u * 64u, rows16 = ((uint64_t)B + 15u) / 16u;
-  if (tiles >= 2048u && pad64 * 8u <= rows16 * 16u * 9u) return launch_mfma<32, 2, 2>(a, s);
+  const bool long_rows = h >= 160u || (h > 64u && V <= 40000u);
+  if (long_rows && tiles >= 2048u && pad64 * 8u <= rows16 * 16u * 9u) return launch_mfma<32, 2, 2>(a, s);
   // Pairs of 16-row tiles share a workgroup's part of embed; an odd count
   // would pad (24 rows: 26.6 us one by one, 25.3 in a pair; 48: 37.8, 44.0).
   return rows16 % 2u ? launch_mfma<16, 1, 4>(a, s) : launch_mfma<16, 2, 2>(a, s);

@@ -133,7 +133,10 @@ def test_one_hot_hidden_rows_select_embedding_columns(sampler):
 @pytest.mark.parametrize("B,V,h", [
     (1, 33, 0), (1, 31, 4), (1, 16385, 129), (2, 1000, 1027), (2, 33, 127), (3, 16384, 36), (3, 16388, 40), (4, 65, 1156),
     (4, 16385, 32), (5, 64, 33), (16, 65, 35), (17, 63, 64), (32, 129, 31), (33, 4100, 68), (48, 32768, 12),
-    (49, 32768, 8), (63, 32769, 37), (64, 32767, 100), (65, 70001, 5), (96, 2049, 64), (128, 16353, 63)])
+    (49, 32768, 8), (63, 32769, 37), (64, 32767, 100), (65, 70001, 5), (96, 2049, 64), (128, 16353, 63),
+    (8, 65535, 16), (8, 65536, 16), (7, 80000, 4), (33, 16001, 3), (64, 31249, 17), (64, 31250, 17), (63, 40000, 48),
+    (97, 20641, 48), (65, 32769, 49), (255, 62500, 64), (256, 62500, 64), (8, 600001, 5), (33000, 64, 4),
+    (63, 32769, 165), (65, 70001, 160), (65, 70001, 159), (65, 40000, 65), (65, 40001, 65), (66, 39997, 64), (128, 16353, 191), (64, 32767, 228)])
 def test_kernel_boundaries(sampler, B, V, h):
     rs = np.random.default_rng(B * 131 + V + h)
     hidden, embed = _case(rs, B, V, h, scale=0.3)
@@ -173,3 +176,53 @@ def test_rows_off_16_byte_alignment_and_extreme_products(sampler, B):
     want = oracle.linear_fwd(hidden, embed, threads=8)
     assert np.count_nonzero(want) > 0
     assert np.array_equal(lg.cpu().numpy(), want)
+
+
+# One of each kernel: the GEMV, 16 x 16 tiles, 32 x 32 tiles, vector multiplies.
+KERNELS = [(1, 20000, 36), (4, 9000, 36), (20, 9000, 36), (64, 33000, 164), (64, 33000, 12)]
+
+
+def _logits(sampler, hidden, embed):
+    seeds = np.arange(hidden.shape[0], dtype=np.uint64)
+    return _run(sampler, hidden, embed, make_params(0.0, 1, 1.0, 0.0, 1.0), seeds)
+
+
+@pytest.mark.parametrize("B,V,h", KERNELS)
+def test_products_over_random_bit_patterns(sampler, B, V, h):
+    """One nonzero element per row, of any bit pattern (denormals, infinities
+    and NaNs among them): each logit is one product, rounded as binary32
+    multiplies round."""
+    rs = np.random.default_rng(h * V + B)
+    bits = lambda n: rs.integers(0, 2**32, n, dtype=np.uint64).astype(np.uint32).view(np.float32)  # noqa: E731
+    hidden, embed = np.zeros((B, h), dtype=np.float32), np.zeros((V, h), dtype=np.float32)
+    k = int(rs.integers(0, h))
+    hidden[:, k], embed[:, k] = bits(B), bits(V)
+    hidden[0, k] = np.float32(1e-42)  # a denormal among any number of rows
+    embed[:4, k] = np.inf, -np.inf, np.nan, np.float32(3e-45)
+    lg = _logits(sampler, hidden, embed)[3]
+    with np.errstate(all="ignore"):
+        want = hidden[:, k][:, None] * embed[:, k][None, :]
+    # (0 * inf and 0 * NaN stay in the column's own accumulator: no other
+    # element of a row is infinite.)
+    assert np.array_equal(np.isnan(lg), np.isnan(want))
+    assert np.array_equal(lg[~np.isnan(lg)], want[~np.isnan(want)])
+
+
+@pytest.mark.parametrize("B,V,h", KERNELS)
+def test_infinities_and_nans_stay_in_their_rows(sampler, B, V, h):
+    """Infinite and NaN elements of some hidden and embedding rows: those rows'
+    and outputs' logits are the oracle's, and so are the greedy ids."""
+    rs = np.random.default_rng(h + V + B)
+    hidden, embed = _case(rs, B, V, h, scale=0.3)
+    hidden[::3, rs.integers(0, h)] = np.inf
+    hidden[2::5, rs.integers(0, h)] = -np.inf
+    hidden[4::7, rs.integers(0, h)] = np.nan
+    at = rs.choice(V, 60, replace=False)
+    embed[at[:20], rs.integers(0, h)] = np.inf
+    embed[at[20:40], rs.integers(0, h)] = -np.inf
+    embed[at[40:], rs.integers(0, h)] = np.nan
+    ids, _, _, lg = _logits(sampler, hidden, embed)
+    want = oracle.linear_fwd(hidden, embed, threads=8)
+    assert np.array_equal(lg, want, equal_nan=True)
+    o = oracle.sample_batch(want, make_params(0.0, 1, 1.0, 0.0, 1.0), np.arange(B, dtype=np.uint64), V=V, threads=8)
+    assert np.array_equal(ids, o.ids)
