@@ -150,7 +150,7 @@ int llmhip_sample_device(llmhip_ctx* ctx, const float* logits, size_t B, size_t 
  * scratch go into one array of LLMHIP_NOALLOC_SCRATCH_BYTES that the library
  * holds on each GPU it runs on, until the process ends. A call needs
  *   ceil(((B - 1) * params_stride + 1) * 20 / 256) * 256   (params, if per row)
- *   + 4096                                                 (reserved)
+ *   + 4096                                                 (unused)
  *   + B * w * Vp * 4                                       (scratch)
  * bytes, with Vp = V rounded up to 1024 and w = 2 when every row is greedy
  * or has 0 < top_k <= 4096, top_k < V, else 5. A larger call returns

@@ -1200,12 +1200,9 @@ __device__ __forceinline__ bool fast_row(const SampleArgs& a, FastLds<NCH, BIGK>
     reinterpret_cast<uint4*>(L.fine)[tid] = make_uint4(0u, 0u, 0u, 0u);
     lds_barrier();  // every wave has read the candidate count and overflow flag above
     LLMHIP_MARK(11);
-    if (tid == 0) {
-      L.misc[kCandN] = 0u;
-      L.misc[kOverflow] = 0u;
-    }
+    if (tid == 0) L.misc[kCandN] = 0u;
     slot_n = kCandN;
-    slot_o = kOverflow;
+    slot_o = kOverflow;  // (never set below: the scan takes what the entries hold)
     float kmx = -INFINITY;  // this thread's known maximum
     if (by_chunk) {
 #pragma unroll
@@ -1291,9 +1288,9 @@ __device__ __forceinline__ bool fast_row(const SampleArgs& a, FastLds<NCH, BIGK>
       LLMHIP_MARK(13);
       n = L.misc[kCandN];
     }
-    if (__builtin_expect(huge || n > ncap || L.misc[kOverflow] != 0u, 0)) {
-      // Too many values at or above the threshold for the scan entries or
-      // the list (a large K): narrow it per slot. Level 1: the fine bin
+    if (__builtin_expect(huge || n > ncap, 0)) {
+      // Too many values at or above the threshold for the list (a large K):
+      // narrow it per slot. Level 1: the fine bin
       // holding the K-th largest known value at or above it (tk0 <= t0, so
       // at least K are). Level 2, when that bin is
       // crowded: 12 more key bits inside it. At least K final values lie at
@@ -1302,7 +1299,7 @@ __device__ __forceinline__ bool fast_row(const SampleArgs& a, FastLds<NCH, BIGK>
       uint32_t* fine1 = reinterpret_cast<uint32_t*>(L.ent);  // kWaves * kEnt float4 >= kFineBins words
       uint32_t* coarse1 = L.etag;                              // kWaves * kEnt words >= kCoarseBins
       reinterpret_cast<uint4*>(fine1)[tid] = make_uint4(0u, 0u, 0u, 0u);
-      lds_barrier();  // every wave has read the count and flag, and is past the entries
+      lds_barrier();  // every wave has read the count, and is past the entries
       // (A fresh copy of the mask per loop: shared between the loops, its 32
       // per-slot bits would stay live in registers from one to the next.)
       uint32_t kn1 = known;

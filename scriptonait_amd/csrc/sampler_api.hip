@@ -16,8 +16,9 @@
 // Device memory of llmhip_sample_device_noalloc, for callers that cannot
 // allocate: each GPU the library runs on holds its own copy of this array
 // until the process ends. One call lays out, from the start: the per-row
-// parameters (when params_stride != 0), kBlock reserved words, and the per-row
-// scratch of the sorting path. Host code never passes `scratch` itself to a kernel or a copy (in
+// parameters (when params_stride != 0), kBlock words that nothing uses (the
+// header's formula counts them, and the calls it refuses stay the same), and the
+// per-row scratch of the sorting path. Host code never passes `scratch` itself to a kernel or a copy (in
 // host code the name is a host-side stand-in, not a device address): it uses
 // the address hipGetSymbolAddress returns for the current device, looked up
 // once per device when the first context on that device is created.
@@ -596,7 +597,7 @@ int llmhip_sample_device_noalloc(llmhip_ctx* ctx, const float* logits, size_t B,
                        : std::string("no-alloc scratch: no device address for this device");
     return LLMHIP_ERR_HIP;
   }
-  // The call's layout in the array: params | reserved | per-row scratch.
+  // The call's layout in the array: params | unused | per-row scratch.
   const size_t pbytes =
       params_stride ? (((B - 1) * params_stride + 1) * sizeof(llmhip_params) + 255u) / 256u * 256u : 0u;
   const size_t mbytes = kBlock * sizeof(uint32_t);

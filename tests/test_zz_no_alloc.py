@@ -1,8 +1,7 @@
 """GPU: llmhip_sample_device_noalloc against llmhip_sample_device.
 
 The no-alloc entry runs the same kernels as llmhip_sample_device, with its
-device memory (per-row parameters, the allowed mask's slot layout, the
-sorting path's per-row scratch) taken from the library's fixed per-GPU array
+device memory (per-row parameters and the sorting path's per-row scratch) taken from the library's fixed per-GPU array
 instead of the context's buffers. Three calls in a row, each smaller than
 the last and of another kind, must give the same ids, RNG states, kept counts and
 probabilities as llmhip_sample_device on the same inputs: the array keeps the
