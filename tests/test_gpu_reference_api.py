@@ -111,32 +111,58 @@ def test_generation_loop_with_windowed_history():
         tokens.append(got)
 
 
-@pytest.mark.parametrize("B,V,ld", [(1, 1, 1), (1, 3, 3), (1, 32000, 32000), (3, 32769, 32771), (64, 32000, 32000),
-                                    (65, 32000, 32004), (5, 4099, 5000)])
-@pytest.mark.parametrize("top_k,per_row", [(40, False), (0, False), (2000, True)])
-def test_host_calls_on_both_sides_of_the_staging_limit(sampler, B, V, ld, top_k, per_row):
-    """The host entry gathers small calls in pinned memory and copies larger
-    ones part by part (64 rows of 32000 lie on one side, 65 on the other):
-    dense and strided rows, every kernel, shared and per-row parameters; a
-    second call on other inputs sees only its own."""
+def _host_call_matches(sampler, rs, B, V, ld, top_k, per_row, beyond):
+    """One host call on fresh inputs, against the oracle."""
     from oracle import oracle
     from scriptonait_amd.workloads import PARAMS_DTYPE
 
+    x = rs.standard_normal((B, ld)).astype(np.float32) * 2
+    H = int(rs.integers(0, 200))
+    hist = rs.integers(0, V + 2, B * H).astype(np.uint32)
+    offs = (np.arange(B + 1) * H).astype(np.uint32)
+    allowed = (rs.random(V + beyond) < 0.8).astype(np.uint8)
+    prm = np.zeros(B if per_row else 1, dtype=PARAMS_DTYPE)
+    prm["temperature"], prm["top_k"], prm["top_p"], prm["repetition_penalty"] = 0.8, top_k, 0.95, 1.1
+    if per_row:
+        prm["temperature"][::3] = 0.0
+        prm["top_k"][1::3] = 30
+    seeds = rs.integers(0, 2**63, size=B, dtype=np.uint64)
+    g = sampler.sample_host(x, prm, seeds, hist, offs, allowed=allowed, V=V)
+    o = oracle.sample_batch(x, prm, seeds, hist, offs, allowed=allowed, V=V, threads=8)
+    assert np.array_equal(g.ids, o.ids)
+    assert np.array_equal(g.kept, o.kept)
+    assert np.array_equal(g.rng_state, o.rng_state)
+
+
+@pytest.mark.parametrize("B,V,ld", [(1, 1, 1), (1, 3, 3), (1, 32000, 32000), (3, 32769, 32771), (64, 32000, 32000),
+                                    (65, 32000, 32004), (66, 32000, 32000), (66, 32000, 32004), (5, 4099, 5000)])
+@pytest.mark.parametrize("top_k,per_row", [(40, False), (0, False), (2000, True)])
+def test_host_calls_on_both_sides_of_the_staging_limit(sampler, B, V, ld, top_k, per_row):
+    """The host entry gathers calls of at most 8 MiB in pinned memory and
+    copies larger ones part by part (the logits of 66 rows of 32000 alone are
+    more): dense and strided rows, every kernel, shared and per-row parameters;
+    a second call on other inputs sees only its own."""
     rs = np.random.default_rng(B * V + top_k)
     for call in range(2):
-        x = rs.standard_normal((B, ld)).astype(np.float32) * 2
-        H = int(rs.integers(0, 200))
-        hist = rs.integers(0, V + 2, B * H).astype(np.uint32)
-        offs = (np.arange(B + 1) * H).astype(np.uint32)
-        allowed = (rs.random(V + 1 - call) < 0.8).astype(np.uint8)
-        prm = np.zeros(B if per_row else 1, dtype=PARAMS_DTYPE)
-        prm["temperature"], prm["top_k"], prm["top_p"], prm["repetition_penalty"] = 0.8, top_k, 0.95, 1.1
-        if per_row:
-            prm["temperature"][::3] = 0.0
-            prm["top_k"][1::3] = 30
-        seeds = rs.integers(0, 2**63, size=B, dtype=np.uint64)
-        g = sampler.sample_host(x, prm, seeds, hist, offs, allowed=allowed, V=V)
-        o = oracle.sample_batch(x, prm, seeds, hist, offs, allowed=allowed, V=V, threads=8)
-        assert np.array_equal(g.ids, o.ids)
-        assert np.array_equal(g.kept, o.kept)
-        assert np.array_equal(g.rng_state, o.rng_state)
+        _host_call_matches(sampler, rs, B, V, ld, top_k, per_row, 1 - call)
+
+
+def test_host_calls_alternate_across_the_staging_limit(sampler):
+    """Staged and copied calls in turn on one context, which hands its flag
+    word from one kind to the other. Each is followed by one whose waits may
+    spin once only: that one reports a timeout or returns, and the next call,
+    of the other kind, does not see its flags."""
+    from scriptonait_amd import sampler as smp
+
+    rs = np.random.default_rng(17)
+    with smp.Sampler(0) as s:
+        for B, top_k in ((2, 40), (66, 40), (1, 0), (67, 40), (66, 0), (3, 2000), (66, 40), (2, 40)):
+            _host_call_matches(s, rs, B, 32000, 32000, top_k, False, 1)
+            s.debug(smp.DEBUG_SPIN_LIMIT, 1)
+            try:
+                s.sample_host(rs.standard_normal((B, 32000)).astype(np.float32), SamplingConfig().to_params(),
+                              np.arange(B, dtype=np.uint64), V=32000)
+            except smp.SamplerError as e:
+                assert e.status == -3
+            finally:
+                s.debug(smp.DEBUG_SPIN_LIMIT, 0)

@@ -12,6 +12,19 @@ from scriptonait_amd.workloads import make_params
 pytestmark = pytest.mark.gpu
 
 
+# K past 384, whose threshold comes from the chunks' maxima (and its scan, in
+# rounds, lists more than the small-K kernel ranks), up to 1024 and just past it,
+# where the per-slot narrowing takes over.
+LARGE_K = [(8191, 1500, 5), (16384, 2500, 4), (32000, 1000, 12), (32000, 4000, 3), (32768, 3000, 5)]
+
+
+@pytest.mark.parametrize("V,top,reps", LARGE_K)
+@pytest.mark.parametrize("K", [385, 700, 1024, 1025])
+@pytest.mark.parametrize("masked", [False, True])
+def test_every_top_id_penalized_at_large_k(sampler, V, top, reps, K, masked):
+    test_every_top_id_penalized(sampler, V, top, reps, K, masked)
+
+
 @pytest.mark.parametrize("V,top,reps", [(4096, 300, 12), (8191, 500, 12), (16384, 700, 9), (32000, 400, 12),
                                         (32000, 1000, 12), (32768, 1500, 12), (32000, 2500, 7)])
 @pytest.mark.parametrize("K", [1, 20, 40, 64, 100, 380])
