@@ -32,13 +32,15 @@
 //     folds and the draw (draw_tail_bcast for K <= 64, draw_tail_lds
 //     above), while the other waves issue the next row's loads.
 //
-// Rows of a large K raise the threshold after every two pieces: a histogram
-// of the unmarked values listed so far, in bins of 1/512 of a value, gives
-// their K-th largest, and the row's last one cuts the list to little more than
-// K before the sort. (From the first threshold alone a row lists 1.2-1.4 K
-// values per 32768, so 512 rows of 131072 at top_k 1000 did not fit the list
-// and took the sorting path: 327 us, and 98 so. 1024 rows of 50257 at top_k 1000,
-// which fitted: 176.5 -> 173.)
+// Rows of a large K (stream_refines) raise the threshold after every two
+// pieces: a histogram of the unmarked values listed so far, in bins of 1/512 of
+// a value, gives their K-th largest, and the row's last one cuts the list to
+// little more than K before the sort. (From the first threshold alone a row lists
+// 1.2-1.4 K values per 32768, so 512 rows of 131072 at top_k 1000 did not fit the
+// list and took the sorting path: 327 us, and 98 so.) A list of more than 3072
+// drops what the raised threshold leaves below it on the way: values tied at the
+// threshold would overflow it otherwise (the same rows rounded to quarters: 303 of
+// them handed over, 250 us, and 112 so).
 //
 // A row the list cannot hold (about 1.2 K values per 32768 of the row are
 // listed), whose threshold is not bounded this way (fewer than K finite
