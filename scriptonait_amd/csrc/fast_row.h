@@ -75,9 +75,15 @@ constexpr uint32_t kTauWaves = 8;                 // waves whose maxima form the
 constexpr uint32_t kSpecNum = 8, kSpecDen = 5;    // the threshold aims at ~(kSpecNum/kSpecDen)*K values
 // Fewer than K / 32 survivors: the second speculative pass, four times as deep
 // at most, would find too few as well (4 us for a row of a saturated window),
-// and the proven threshold follows at once.
-constexpr bool second_pass_pays(uint32_t n, uint32_t K) { return n * 32u >= K; }
-static_assert(!second_pass_pays(0u, 1u) && second_pass_pays(1u, 32u) && !second_pass_pays(1u, 33u), "at every K");
+// and the proven threshold follows at once. With a count table that threshold
+// reads the table for the whole row, and the pass is worth its try from K = 32
+// on: 256 rows of 32000 at K = 64, a window of 4096 that 150 steps have filled
+// in part 15.7 us with it and 18.2 without, one full of the row's own draws 28.8
+// and 25.2 (48 before there was a rule); at K = 20 21.7 and 19.0, 22.2 and 19.7.
+constexpr bool second_pass_pays(uint32_t n, uint32_t K, bool counts) { return n * 32u >= K || (counts && K >= 32u); }
+static_assert(!second_pass_pays(0u, 1u, false) && second_pass_pays(1u, 32u, false) && !second_pass_pays(1u, 33u, false) &&
+                  !second_pass_pays(0u, 31u, true) && second_pass_pays(0u, 32u, true),
+              "at every K");
 constexpr uint32_t kSpecMaxK = 384;               // larger K: the scan entries would overflow; proven threshold
 constexpr uint32_t kRefineCount = 16;             // a fine bin holding more keys is split once more
 constexpr uint32_t kSortedK = 1024;               // K up to which the sorted top K is copied to skey/sid
@@ -1151,7 +1157,7 @@ __device__ __forceinline__ bool fast_row(const SampleArgs& a, FastLds<NCH, BIGK>
   // deep enough for the 5K/4 - n survivors still missing (at most 8 times
   // the first). One wave selects it (a selection in every wave would compete
   // for the ALUs).
-  if (__builtin_expect(spec && n < K && second_pass_pays(n, K) && !ovf, 0)) {
+  if (__builtin_expect(spec && n < K && second_pass_pays(n, K, CMODE) && !ovf, 0)) {
     if (wave == 0u) {
       __builtin_amdgcn_s_setprio(3);  // as for the first threshold
       const uint64_t q = spec_q(L.misc[kSampled]);
